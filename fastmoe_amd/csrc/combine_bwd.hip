@@ -14,10 +14,15 @@
 // grad_w needs no cross-wave reduction: a wave owns whole rows and reduces its dot product with a
 // xor butterfly.  Segment T of the plan (rows whose scatter index was out of range) gets zeros.
 //
-// Two passes.  When both gradients are wanted the grad_X pass (a write stream) and the grad_w pass
-// (read streams only) run as two back-to-back launches rather than one fused kernel: HBM loses
+// Two passes.  When both gradients are wanted the grad_w pass (read streams only) and the grad_X
+// pass (a write stream) run as two back-to-back launches rather than one fused kernel: HBM loses
 // about a tenth of its throughput when a kernel interleaves this much reading and writing at fine
 // grain, which costs more than reading grad_out (T * D, one k-th of X at top-k) a second time.
+// The grad_w pass goes first: it leaves grad_out in the Infinity Cache (256 MB; X is read
+// non-temporally), so that the grad_X pass writes without HBM reads in between.  bf16, T=4096,
+// D=16384, top-8, three sets of buffers in turn, after the forward: grad_w 191 + grad_X 218 us,
+// against grad_X 255 + grad_w 180 us in the other order (on one set of buffers, which the previous
+// step leaves in the cache, both orders take 175 + 210 us).
 #include "plan.h"
 
 namespace fmoe {
@@ -347,9 +352,9 @@ static int launch_bwd_x(const BwdArgs& a) {
   const bool fused = fmoe_host::opt(fmoe_host::kOptBwdFused) != 0;
   if (!vec_ok) {
     if (a.gx && a.gw && fused) return launch_bwd_k<TX, 1, 4, true, true>(a);
-    if (a.gx)
-      if (int rc = launch_bwd_k<TX, 1, 4, true, false>(a)) return rc;
-    return a.gw ? launch_bwd_k<TX, 1, 4, false, true>(a) : FMOE_OK;
+    if (a.gw)
+      if (int rc = launch_bwd_k<TX, 1, 4, false, true>(a)) return rc;
+    return a.gx ? launch_bwd_k<TX, 1, 4, true, false>(a) : FMOE_OK;
   }
   const int64_t row_bytes = a.D * eb;
   int ux = (int)fmoe_host::opt(fmoe_host::kOptBwdU);
@@ -359,9 +364,9 @@ static int launch_bwd_x(const BwdArgs& a) {
     uw = row_bytes >= 24576 ? 4 : (row_bytes >= 4096 ? 2 : 1);
   }
   if (a.gx && a.gw && fused) return launch_bwd_v<TX, V, true, true>(a, ux);
-  if (a.gx)
-    if (int rc = launch_bwd_v<TX, V, true, false>(a, ux)) return rc;  // grad_X: write pass
-  return a.gw ? launch_bwd_v<TX, V, false, true>(a, uw) : FMOE_OK;    // grad_w: read pass
+  if (a.gw)
+    if (int rc = launch_bwd_v<TX, V, false, true>(a, uw)) return rc;  // grad_w: read pass
+  return a.gx ? launch_bwd_v<TX, V, true, false>(a, ux) : FMOE_OK;    // grad_X: write pass
 }
 
 }  // namespace fmoe

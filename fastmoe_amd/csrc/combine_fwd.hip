@@ -34,7 +34,7 @@ template <typename TX, typename TO, int V, int U, int RB, bool AL>
 __device__ __forceinline__ void fwd_det_body(const int32_t* __restrict__ row_ptr,
                                              const Rec* __restrict__ rec, TO* __restrict__ out,
                                              int64_t out_stride, uint32_t D, uint32_t t,
-                                             uint32_t chunk, int accumulate) {
+                                             uint32_t chunk, int accumulate, int out_stream) {
   using VX = Vec<TX, V>;
   using VO = Vec<TO, V>;
   using raw_t = typename VX::raw_t;
@@ -103,9 +103,14 @@ __device__ __forceinline__ void fwd_det_body(const int32_t* __restrict__ row_ptr
       }
     }
   }
+  // columns >= D: dropped by range check
+  if (out_stream) {  // wave-uniform
 #pragma unroll
-  for (int u = 0; u < U; ++u)  // columns >= D: dropped by range check
-    VO::template st<FMOE_OUT_CPOL>(ro, ooff[u], acc[u]);
+    for (int u = 0; u < U; ++u) VO::template st<kCPol>(ro, ooff[u], acc[u]);
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u) VO::template st<FMOE_OUT_CPOL>(ro, ooff[u], acc[u]);
+  }
 }
 
 template <typename TX, typename TO, int V, int U, int RB>
@@ -114,7 +119,7 @@ __global__ __launch_bounds__(kGroup) void k_fwd_det(const int32_t* __restrict__ 
                                                     const Rec* __restrict__ rec,
                                                     TO* __restrict__ out, int64_t out_stride,
                                                     uint32_t D, uint32_t T, uint32_t chunks,
-                                                    int accumulate) {
+                                                    int accumulate, int out_stream) {
   const bool al = !(V > 1 && status[kStatusMisaligned] != 0);
   const uint32_t units = T * chunks;
   // Wave units (token, column chunk); a grid smaller than units / 4 strides over them.
@@ -123,10 +128,11 @@ __global__ __launch_bounds__(kGroup) void k_fwd_det(const int32_t* __restrict__ 
     const uint32_t t = unit / chunks;
     const uint32_t chunk = unit - t * chunks;
     if (al)
-      fwd_det_body<TX, TO, V, U, RB, true>(row_ptr, rec, out, out_stride, D, t, chunk, accumulate);
+      fwd_det_body<TX, TO, V, U, RB, true>(row_ptr, rec, out, out_stride, D, t, chunk, accumulate,
+                                           out_stream);
     else
-      fwd_det_body<TX, TO, V, U, RB, false>(row_ptr, rec, out, out_stride, D, t, chunk,
-                                            accumulate);
+      fwd_det_body<TX, TO, V, U, RB, false>(row_ptr, rec, out, out_stride, D, t, chunk, accumulate,
+                                            out_stream);
   }
 }
 
@@ -546,6 +552,24 @@ struct FwdArgs {
   hipStream_t s;
 };
 
+// Output bytes from which the deterministic forward stores its output non-temporally.  Stored with
+// the temporal policy (FMOE_OUT_CPOL), the output stays dirty in the 256 MB Infinity Cache: the
+// forward itself is up to 5 % shorter, but its lines are written back during the kernels that
+// follow, which loses more once the output is a large part of that cache.  Measured on one MI355X
+// with three sets of buffers in turn (bf16, us per call; temporal / non-temporal):
+//   T, D, k (output)             forward          forward + backward
+//   8192, 4096, 6 (64 MiB)       77.6 /  81.2     246.0 / 228.6
+//   2048, 16384, 8 (64 MiB)     100.0 / 101.6     313.7 / 297.5
+//   3072, 16384, 8 (96 MiB)     164.2 / 159.6     469.4 / 451.7
+//   4096, 16384, 8 (128 MiB)    217.2 / 212.2     635.9 / 613.4
+//   16384, 4096, 6 (128 MiB)    167.1 / 160.0     483.8 / 463.8
+//   6144, 16384, 8 (192 MiB)    324.4 / 319.7     930.4 / 922.9
+// The line lies where the forward alone gains too; below it a program that only runs forwards
+// keeps the shorter one.  An accumulating call has just read its output and the caller has just
+// written it, so its lines are in the cache: fp32, 256 MiB, zero-fill + call 291.6 us temporal,
+// 316.9 us non-temporal; it stays temporal.
+constexpr int64_t kOutStreamBytes = int64_t(96) << 20;
+
 template <typename TX, typename TO, int V, int U, int RB>
 static int launch_fwd_k(const FwdArgs& a, int64_t chunks) {
   unsigned blocks;
@@ -555,7 +579,8 @@ static int launch_fwd_k(const FwdArgs& a, int64_t chunks) {
     if (persist > 0 && (unsigned)persist < blocks) blocks = (unsigned)persist;
     hipLaunchKernelGGL((k_fwd_det<TX, TO, V, U, RB>), dim3(blocks), dim3(kGroup), 0, a.s, a.status,
                        a.row_ptr, a.rec, static_cast<TO*>(a.out), a.out_stride, (uint32_t)a.D,
-                       (uint32_t)a.T, (uint32_t)chunks, a.accumulate);
+                       (uint32_t)a.T, (uint32_t)chunks, a.accumulate,
+                       !a.accumulate && a.T * a.D * (int64_t)sizeof(TO) >= kOutStreamBytes);
     return fmoe_host::check_launch("fmoe_combine_fwd(det)");
   }
   if constexpr (V == 1 && sizeof(TO) == 2) {

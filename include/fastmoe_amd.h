@@ -298,7 +298,7 @@ FMOE_API int fmoe_combine_fwd_noalloc(const int64_t* host_ptrs, const int64_t* h
  *              NULL to skip it.  grad_X[g] = round_x(f32(grad_out[idx[g]]) * w[g]).
  * d_grad_w   : [N] of gw_dtype, or NULL to skip it (then the expert buffers are not read).
  *              grad_w[g] accumulates the D products in fp64 and rounds once.
- * Given both outputs, the call enqueues two kernels: the grad_X pass, then the grad_w pass.
+ * Given both outputs, the call enqueues two kernels: the grad_w pass, then the grad_X pass.
  */
 FMOE_API int fmoe_combine_bwd(const void* d_plan, int64_t num_rows, int64_t num_tokens, int64_t hidden,
                      int x_dtype, const void* d_grad_out, int gout_dtype, int64_t gout_row_stride,
