@@ -94,6 +94,10 @@ SIGNATURES: dict[str, tuple] = {
     ),
     "fmoe_permute_gather": (_c_int, [_c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_vp, _c_vp]),
     "fmoe_permute_gate_grad": (_c_int, [_c_vp, _c_i64, _c_vp, _c_int, _c_vp, _c_vp]),
+    "fmoe_permute_backward": (
+        _c_int,
+        [_c_vp, _c_i64, _c_i64, _c_i64, _c_int, _c_vp, _c_vp, _c_vp, _c_int, _c_vp, _c_vp],
+    ),
 }
 
 _LIB: ctypes.CDLL | None = None

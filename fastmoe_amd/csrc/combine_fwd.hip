@@ -28,6 +28,40 @@
 
 namespace fmoe {
 
+// acc += w[i] * row i, for the cnt records of a batch held one per lane, in record order: R rows of
+// U vectors per lane in flight.  The spare slots of a partial batch load through an empty range
+// (num_records 0): the hardware range check returns zeros without a memory request, so every load
+// is issued unconditionally and none is wasted.
+template <typename TX, int V, int U, int R, bool AL>
+__device__ __forceinline__ void add_rows(const LaneRecs& lr, int cnt, uint32_t xrow_bytes,
+                                         const uint32_t (&xoff)[U], float (&acc)[U][V]) {
+  using VX = Vec<TX, V>;
+  for (int i = 0; i < cnt; i += R) {
+    typename VX::raw_t a[R][U];
+    float wr[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int ir = min(i + r, cnt - 1);
+      const rsrc_t rx = make_rsrc(lr.src(ir), i + r < cnt ? xrow_bytes : 0u);
+      wr[r] = lr.w(ir);
+#pragma unroll
+      for (int u = 0; u < U; ++u) a[r][u] = load_x<TX, V, AL>(rx, xoff[u]);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (i + r < cnt) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          float x[V];
+          VX::cvt(a[r][u], x);
+#pragma unroll
+          for (int v = 0; v < V; ++v) acc[u][v] = acc[u][v] + x[v] * wr[r];
+        }
+      }
+    }
+  }
+}
+
 // Tile of one wave unit: U 16-byte vectors per lane per row (64 * V * U columns) and batches of
 // R rows, so R * U independent loads per lane are in flight before the first use.
 template <typename TX, typename TO, int V, int U, int RB, bool AL>
@@ -35,9 +69,7 @@ __device__ __forceinline__ void fwd_det_body(const int32_t* __restrict__ row_ptr
                                              const Rec* __restrict__ rec, TO* __restrict__ out,
                                              int64_t out_stride, uint32_t D, uint32_t t,
                                              uint32_t chunk, int accumulate, int out_stream) {
-  using VX = Vec<TX, V>;
   using VO = Vec<TO, V>;
-  using raw_t = typename VX::raw_t;
   constexpr int CW = kWave * V * U;
   // The misaligned-row path (element loads) takes one row at a time so that it does not set the
   // register budget of the kernel.
@@ -74,34 +106,7 @@ __device__ __forceinline__ void fwd_det_body(const int32_t* __restrict__ row_ptr
     // A segment of up to 64 rows comes unordered from the plan: order it by g here.  Longer
     // segments are already in ascending g.
     if (end - beg <= kWave) lr.sort_by_row(cnt, lane);
-    for (int i = 0; i < cnt; i += R) {
-      // Batch of R rows.  The spare slots of a partial batch load through an empty range
-      // (num_records 0): the hardware range check returns zeros without a memory request, so
-      // every load is issued unconditionally and none is wasted.
-      raw_t a[R][U];
-      float wr[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int ir = min(i + r, cnt - 1);
-        const rsrc_t rx = make_rsrc(lr.src(ir), i + r < cnt ? xrow_bytes : 0u);
-        wr[r] = lr.w(ir);
-#pragma unroll
-        for (int u = 0; u < U; ++u) a[r][u] = load_x<TX, V, AL>(rx, xoff[u]);
-      }
-      // Adds in ascending row order (the order of the plan segment).
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (i + r < cnt) {
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            float x[V];
-            VX::cvt(a[r][u], x);
-#pragma unroll
-            for (int v = 0; v < V; ++v) acc[u][v] = acc[u][v] + x[v] * wr[r];
-          }
-        }
-      }
-    }
+    add_rows<TX, V, U, R, AL>(lr, cnt, xrow_bytes, xoff, acc);
   }
   // columns >= D: dropped by range check
   if (out_stream) {  // wave-uniform
@@ -136,6 +141,66 @@ __global__ __launch_bounds__(kGroup) void k_fwd_det(const int32_t* __restrict__ 
   }
 }
 
+// ---- backward of the dispatch permutation ------------------------------------------------------
+// grad_x[t, :] = sum of the packed-row gradients of token t's k slots, in ascending packed-row
+// order, and (GATES) grad_gates[i] = grad_sorted[slot_pos[i]].  The slot map is the token-major
+// inverse already: slot t * k + j sits at packed row slot_pos[t * k + j] of one buffer, so a wave
+// makes its records in registers from one load and the combine needs no plan, no unit gates and no
+// launch but this one.  A wave owns a (token, column chunk) and sums with k_fwd_det's arithmetic
+// (unit gates: x * 1), so the result is the planned combine's bit for bit; the wave of chunk 0
+// moves the token's gate gradients.  A slot_pos entry outside [0, N) adds nothing.
+// Bound by HBM like k_fwd_det.  T=8192, D=4096, top-6, bf16, permutation and its backward: 195.6 us
+// with the slot-map plan, the combine and the gate-gradient kernel (and autograd's fills of the
+// integer outputs' gradients), 184.4 us with this kernel alone.
+template <typename TX, int V, int U, int RB, bool GATES, typename TG>
+__global__ __launch_bounds__(kGroup) void k_slots_bwd(const int32_t* __restrict__ slot_pos,
+                                                      uint32_t k, uint32_t N,
+                                                      const TX* __restrict__ rows, uint32_t D,
+                                                      uint32_t T, uint32_t chunks,
+                                                      TX* __restrict__ out, int out_stream,
+                                                      const TG* __restrict__ gates,
+                                                      TG* __restrict__ grad_gates) {
+  using VX = Vec<TX, V>;
+  constexpr int CW = kWave * V * U;
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint32_t unit = blockIdx.x * kWavesPerGroup + (uint32_t)uniform(threadIdx.x / kWave);
+  const uint32_t t = unit / chunks;
+  if (t >= T) return;  // wave-uniform
+  const uint32_t chunk = unit - t * chunks;
+  const uint32_t row_bytes = D * (uint32_t)sizeof(TX);
+  const uint32_t slot = t * k + (uint32_t)lane;
+  const bool mine = (uint32_t)lane < k;
+  const uint32_t pos = mine ? (uint32_t)slot_pos[slot] : N;
+  const bool ok = pos < N;  // a negative entry is a large unsigned one
+  if (GATES && chunk == 0 && mine) grad_gates[slot] = ok ? gates[pos] : TG{};
+  LaneRecs lr;
+  lr.g = ok ? (int32_t)pos : 0x7fffffff;  // entries out of range sort behind the others
+  const uint64_t src = (uint64_t)(uintptr_t)rows + (uint64_t)(ok ? pos : 0u) * row_bytes;
+  lr.src_lo = (uint32_t)src;
+  lr.src_hi = (uint32_t)(src >> 32);
+  lr.w_bits = __float_as_uint(1.f);
+  const int cnt = __builtin_popcountll(__ballot(ok));
+  lr.sort_by_row((int)k, lane);
+  uint32_t off[U];
+  float acc[U][V];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    off[u] = (chunk * CW + (uint32_t)lane * V + (uint32_t)u * kWave * V) * (uint32_t)sizeof(TX);
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[u][v] = 0.f;
+  }
+  add_rows<TX, V, U, RB, true>(lr, cnt, row_bytes, off, acc);
+  const rsrc_t ro = make_rsrc(out + (int64_t)t * D, row_bytes);
+  // columns >= D: dropped by range check
+  if (out_stream) {  // wave-uniform
+#pragma unroll
+    for (int u = 0; u < U; ++u) VX::template st<kCPol>(ro, off[u], acc[u]);
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u) VX::template st<FMOE_OUT_CPOL>(ro, off[u], acc[u]);
+  }
+}
+
 // ---- small inputs: the deterministic forward without a plan --------------------------------
 // For at most kSmallRows rows the plan is not worth its own launch.  Every workgroup stages the
 // token id of each row in LDS (-1 for an index outside [0, T)); a wave owns one (token, column
@@ -152,9 +217,7 @@ __global__ __launch_bounds__(kGroup) void k_fwd_small(const HostTable meta,
                                                       uint32_t chunks, TO* __restrict__ out,
                                                       int64_t out_stride, int accumulate,
                                                       int32_t* __restrict__ status) {
-  using VX = Vec<TX, V>;
   using VO = Vec<TO, V>;
-  using raw_t = typename VX::raw_t;
   constexpr int CW = kWave * V * U;
   constexpr int R = AL ? 4 : 1;  // rows per batch of loads (one at a time for element loads)
   __shared__ int tok[kSmallRows];
@@ -232,30 +295,7 @@ __global__ __launch_bounds__(kGroup) void k_fwd_small(const HostTable meta,
         if (lane < rest) win[wave][lane] = carry;
         have = rest;
         seen += cnt;
-        for (int i = 0; i < cnt; i += R) {
-          raw_t a[R][U];
-          float wr[R];
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            const int ir = min(i + r, cnt - 1);
-            const rsrc_t rx = make_rsrc(lr.src(ir), i + r < cnt ? xrow_bytes : 0u);
-            wr[r] = lr.w(ir);
-#pragma unroll
-            for (int u = 0; u < U; ++u) a[r][u] = load_x<TX, V, AL>(rx, xoff[u]);
-          }
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            if (i + r < cnt) {
-#pragma unroll
-              for (int u = 0; u < U; ++u) {
-                float x[V];
-                VX::cvt(a[r][u], x);
-#pragma unroll
-                for (int v = 0; v < V; ++v) acc[u][v] = acc[u][v] + x[v] * wr[r];
-              }
-            }
-          }
-        }
+        add_rows<TX, V, U, R, AL>(lr, cnt, xrow_bytes, xoff, acc);
       }
     }
     if (accumulate && seen == 0) continue;  // nothing routed here: out keeps its contents
@@ -623,16 +663,16 @@ static int launch_fwd_u(const FwdArgs& a) {
 // against the choice by D alone: T=16384, D=7168: k=1 129 -> 75 us, k=2 146 -> 109 us, k=8 355 ->
 // 349 us (Zipf) and 361 -> 354 us (top-k); D=5120, 3072, 6144 at k=8 about 2 % faster; D=4096 and
 // 16384 at k=2, 6 and 8 unchanged.
-static void pick_det_tile(const FwdArgs& a, int V, int* U, int* R) {
-  *U = pick_u(a.D, V);
+static void pick_det_tile(int64_t N, int64_t T, int64_t D, int V, int* U, int* R) {
+  *U = pick_u(D, V);
   *R = *U >= 4 ? 4 : 8;
-  if (fmoe_host::opt(fmoe_host::kOptFwdDetU) != 0 || a.N == 0) return;  // U forced: keep R by U
-  if (2 * a.N <= 3 * a.T && a.D >= (int64_t)kWave * V * 4) {  // r <= 1.5, a whole chunk of 4
+  if (fmoe_host::opt(fmoe_host::kOptFwdDetU) != 0 || N == 0) return;  // U forced: keep R by U
+  if (2 * N <= 3 * T && D >= (int64_t)kWave * V * 4) {  // r <= 1.5, a whole chunk of 4
     *U = 4;
     *R = 2;
-  } else if (a.N <= 3 * a.T) {                                  // r <= 3
+  } else if (N <= 3 * T) {                              // r <= 3
     if (*U >= 2) *R = 4;
-  } else if (a.N >= 7 * a.T && *U == 2) {                       // r >= 7
+  } else if (N >= 7 * T && *U == 2) {                   // r >= 7
     *U = 1;
     *R = 8;
   }
@@ -651,7 +691,7 @@ static int launch_fwd_v(const FwdArgs& a) {
     if (!((U == 4 && (R == 4 || R == 2)) || (U == 2 && (R == 8 || R == 4)) ||
           (U == 1 && R == 8))) {
       if (a.mode == FMOE_MODE_DET) {
-        pick_det_tile(a, V, &U, &R);
+        pick_det_tile(a.N, a.T, a.D, V, &U, &R);
       } else {
         U = pick_u(a.D, V);
         R = U >= 4 ? 4 : 8;
@@ -687,6 +727,56 @@ static int launch_fwd_x(const FwdArgs& a, int out_dtype) {
   return FMOE_EINVAL;
 }
 
+
+// The dispatch permutation's backward: k_fwd_det's tiles over the packed-row gradients.
+struct SlotsBwdArgs {
+  const int32_t* slot_pos;
+  int64_t T, k, D;
+  const void* rows;
+  void* out;
+  const void* gates;
+  void* grad_gates;
+  hipStream_t s;
+};
+
+template <typename TX, int V, int U, int RB, bool GATES, typename TG>
+static int launch_slots_bwd_k(const SlotsBwdArgs& a) {
+  const int64_t CW = (int64_t)kWave * V * U;
+  const int64_t chunks = (a.D + CW - 1) / CW;
+  unsigned blocks;
+  if (int rc = grid_for(a.T * chunks, "fmoe_permute_backward", &blocks)) return rc;
+  hipLaunchKernelGGL((k_slots_bwd<TX, V, U, RB, GATES, TG>), dim3(blocks), dim3(kGroup), 0, a.s,
+                     a.slot_pos, (uint32_t)a.k, (uint32_t)(a.T * a.k),
+                     static_cast<const TX*>(a.rows), (uint32_t)a.D, (uint32_t)a.T,
+                     (uint32_t)chunks, static_cast<TX*>(a.out),
+                     a.T * a.D * (int64_t)sizeof(TX) >= kOutStreamBytes,
+                     static_cast<const TG*>(a.gates), static_cast<TG*>(a.grad_gates));
+  return fmoe_host::check_launch("fmoe_permute_backward");
+}
+
+template <typename TX, int V, int U, int RB>
+static int launch_slots_bwd_g(const SlotsBwdArgs& a, int gate_dtype) {
+  if (!a.grad_gates) return launch_slots_bwd_k<TX, V, U, RB, false, uint32_t>(a);
+  if (fmoe_host::dtype_bytes(gate_dtype) == 4)
+    return launch_slots_bwd_k<TX, V, U, RB, true, uint32_t>(a);
+  return launch_slots_bwd_k<TX, V, U, RB, true, uint16_t>(a);
+}
+
+// 16-byte vectors when every row is 16-byte aligned, else one element per lane.
+template <typename TX>
+static int launch_slots_bwd(const SlotsBwdArgs& a, int gate_dtype) {
+  constexpr int V = vec16<TX>();
+  const bool vec_ok = a.D % V == 0 && (uintptr_t)a.rows % 16 == 0 && (uintptr_t)a.out % 16 == 0 &&
+                      fmoe_host::opt(fmoe_host::kOptForceScalar) == 0;
+  if (!vec_ok) return launch_slots_bwd_g<TX, 1, 4, 4>(a, gate_dtype);
+  int U, R;
+  pick_det_tile(a.T * a.k, a.T, a.D, V, &U, &R);
+  if (U == 4 && R == 2) return launch_slots_bwd_g<TX, V, 4, 2>(a, gate_dtype);
+  if (U == 4) return launch_slots_bwd_g<TX, V, 4, 4>(a, gate_dtype);
+  if (U == 2 && R == 4) return launch_slots_bwd_g<TX, V, 2, 4>(a, gate_dtype);
+  if (U == 2) return launch_slots_bwd_g<TX, V, 2, 8>(a, gate_dtype);
+  return launch_slots_bwd_g<TX, V, 1, 8>(a, gate_dtype);
+}
 
 // The small path: a grid of at most kSmallGroups workgroups strides over the (token, chunk) units,
 // so that the ids are staged at most that many times.
@@ -919,4 +1009,34 @@ extern "C" int fmoe_combine_fwd_small(const int64_t* host_ptrs, const int64_t* h
   }
   fmoe_host::set_error("fmoe_combine_fwd_small: bad x dtype %d", x_dtype);
   return FMOE_EINVAL;
+}
+
+extern "C" int fmoe_permute_backward(const int32_t* d_slot_pos, int64_t num_tokens, int64_t top_k,
+                                     int64_t hidden, int dtype, const void* d_grad_rows,
+                                     void* d_grad_x, const void* d_grad_sorted, int gate_dtype,
+                                     void* d_grad_gates, void* stream) {
+  using namespace fmoe;
+  fmoe_host::clear_error();
+  const int64_t T = num_tokens, K = top_k, D = hidden;
+  FMOE_REQUIRE(T >= 1 && K >= 1 && K <= kWave && D >= 1,
+               "fmoe_permute_backward: need T >= 1, D >= 1 and 1 <= top_k <= %d (T=%lld k=%lld "
+               "D=%lld)",
+               kWave, (long long)T, (long long)K, (long long)D);
+  if (T >= (int64_t(1) << 30) || T * K >= (int64_t(1) << 31) || D * 4 >= (int64_t(1) << 31)) {
+    fmoe_host::set_error("fmoe_permute_backward: T*k / D exceed the 32-bit counters");
+    return FMOE_ERANGE;
+  }
+  FMOE_REQUIRE(fmoe_host::is_float_dtype(dtype), "fmoe_permute_backward: bad dtype %d", dtype);
+  FMOE_REQUIRE(d_slot_pos && d_grad_rows && d_grad_x, "fmoe_permute_backward: null device pointer");
+  FMOE_REQUIRE((d_grad_sorted == nullptr) == (d_grad_gates == nullptr),
+               "fmoe_permute_backward: gate gradients need both pointers, or neither");
+  FMOE_REQUIRE(!d_grad_gates || fmoe_host::is_float_dtype(gate_dtype),
+               "fmoe_permute_backward: bad gate dtype %d", gate_dtype);
+  const SlotsBwdArgs a{d_slot_pos, T, K, D, d_grad_rows, d_grad_x, d_grad_sorted, d_grad_gates,
+                       static_cast<hipStream_t>(stream)};
+  switch (dtype) {
+    case FMOE_F32: return launch_slots_bwd<float>(a, gate_dtype);
+    case FMOE_BF16: return launch_slots_bwd<bf16_t>(a, gate_dtype);
+    default: return launch_slots_bwd<f16_t>(a, gate_dtype);
+  }
 }

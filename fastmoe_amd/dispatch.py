@@ -14,12 +14,12 @@ workgroup per token copies its row into its k packed rows).  The packed order is
 within an expert, slots keep ascending order.  The reference's argsort is unstable, so it leaves
 the order of equal ids unspecified; ``torch.argsort(..., stable=True)`` gives exactly this order.
 
-The backward is autograd-complete:
+The backward is autograd-complete (one launch for k <= 64, ``fmoe_permute_backward``):
 * grad of ``permuted_data`` -> grad of ``x_flat``. Each token sums its k packed rows in ascending
   row order, in fp32, rounded once. This is the deterministic combine of this package with unit
   gates: ``reverse_map_indices`` is its scatter index.
 * grad of ``sorted_weights`` -> grad of ``topk_weights``, by the inverse permutation
-  (``fmoe_permute_gate_grad``).
+  (``fmoe_permute_gate_grad`` when it is the only one).
 There is no CPU path: CPU tensors raise.
 """
 from __future__ import annotations
@@ -29,8 +29,7 @@ from typing import NamedTuple, Optional
 import torch
 
 from . import _abi
-from .ops import (_FLOAT_CODES, _INDEX_CODES, _check_experts, _launch_fwd,
-                  _metadata_and_plan_from_slots, _on_device, _refuse_autograd_capture,
+from .ops import (_FLOAT_CODES, _INDEX_CODES, _launch_fwd, _on_device, _refuse_autograd_capture,
                   _require_cuda, _span, _stream_handle, _validate_default,
                   prepare_metadata_and_plan)
 
@@ -68,22 +67,14 @@ def _unit_gates(n: int, dev: torch.device) -> torch.Tensor:
     return ones[:n]
 
 
-def _unit_gate_combine(rows: torch.Tensor, rev: torch.Tensor, slot_pos: torch.Tensor,
-                       num_tokens: int, top_k: int) -> torch.Tensor:
-    """out[t] = sum of rows[g] with rev[g] == t, in ascending g, fp32, rounded once.
-
-    Token t's rows are the packed rows of its slots, slot_pos[t * k + j], so the plan comes from
-    the slot map (one thread per slot) when k <= 64; the forward orders each token's rows by g, so
-    the sum is the same as from the plan of rev."""
+def _unit_gate_combine(rows: torch.Tensor, rev: torch.Tensor, num_tokens: int) -> torch.Tensor:
+    """out[t] = sum of rows[g] with rev[g] == t, in ascending g, fp32, rounded once (the backward
+    of a top-k above 64, which fmoe_permute_backward does not take)."""
     out = torch.empty((num_tokens, rows.shape[1]), dtype=rows.dtype, device=rows.device)
     if rows.shape[0] == 0:
         return out.zero_()
     ones = _unit_gates(rows.shape[0], rows.device)
-    if top_k <= 64 and rows.shape[0] == num_tokens * top_k:
-        meta, plan = _metadata_and_plan_from_slots(_check_experts([rows]), slot_pos, ones,
-                                                   num_tokens, top_k)
-    else:
-        meta, plan = prepare_metadata_and_plan([rows], rev, ones, num_tokens, validate=False)
+    meta, plan = prepare_metadata_and_plan([rows], rev, ones, num_tokens, validate=False)
     _launch_fwd(meta, _abi.MODE_DET, plan, None, None, out, accumulate=False)
     return out
 
@@ -131,7 +122,11 @@ class _TokenPermute(torch.autograd.Function):
         ctx.save_for_backward(rev, slot_pos)
         ctx.num_tokens = T
         ctx.top_k = k
+        ctx.x_dtype, ctx.hidden, ctx.gate_dtype = x_flat.dtype, D, gates.dtype
         ctx.mark_non_differentiable(counts, rev, offsets, slot_pos)
+        # an output without a gradient arrives as None: autograd would otherwise fill a zero tensor
+        # for each of the integer outputs in every backward (four launches)
+        ctx.set_materialize_grads(False)
         return out, sorted_w, counts, rev, offsets, slot_pos
 
     @staticmethod
@@ -139,17 +134,41 @@ class _TokenPermute(torch.autograd.Function):
         rev, slot_pos = ctx.saved_tensors
         _refuse_autograd_capture("the permutation's backward", rev)
         T, k = ctx.num_tokens, ctx.top_k
+        need_x, need_w = ctx.needs_input_grad[:2]
         grad_x = grad_w = None
-        if ctx.needs_input_grad[0] and g_out is not None:
-            grad_x = _unit_gate_combine(g_out.contiguous(), rev, slot_pos, T, k)
-        if ctx.needs_input_grad[1] and g_sorted_w is not None:
-            gs = g_sorted_w.contiguous()
-            grad_w = torch.empty(T * k, dtype=gs.dtype, device=gs.device)
-            with _on_device(gs.device), _span("permute_gate_grad"):
-                rc = _abi.lib().fmoe_permute_gate_grad(
-                    slot_pos.data_ptr(), T * k, gs.data_ptr(), _FLOAT_CODES[gs.dtype],
-                    grad_w.data_ptr(), _stream_handle(gs.device))
-            _abi.check(rc, "fmoe_permute_gate_grad")
+        if need_x:
+            if g_out is None:
+                grad_x = torch.zeros((T, ctx.hidden), dtype=ctx.x_dtype, device=rev.device)
+            elif k <= 64 and rev.numel() > 0 and ctx.hidden > 0:
+                # both gradients in one launch, straight from the slot map
+                rows = g_out.contiguous()
+                gs = g_sorted_w.contiguous() if need_w and g_sorted_w is not None else None
+                grad_x = torch.empty((T, ctx.hidden), dtype=rows.dtype, device=rows.device)
+                if gs is not None:
+                    grad_w = torch.empty(T * k, dtype=gs.dtype, device=gs.device)
+                with _on_device(rows.device), _span("permute_backward"):
+                    rc = _abi.lib().fmoe_permute_backward(
+                        slot_pos.data_ptr(), T, k, ctx.hidden, _FLOAT_CODES[rows.dtype],
+                        rows.data_ptr(), grad_x.data_ptr(),
+                        gs.data_ptr() if gs is not None else None,
+                        _FLOAT_CODES[gs.dtype] if gs is not None else _abi.F32,
+                        grad_w.data_ptr() if gs is not None else None,
+                        _stream_handle(rows.device))
+                _abi.check(rc, "fmoe_permute_backward")
+            else:
+                grad_x = _unit_gate_combine(g_out.contiguous(), rev, T)
+        if need_w and grad_w is None:
+            if g_sorted_w is None:
+                grad_w = torch.zeros(T * k, dtype=ctx.gate_dtype, device=rev.device)
+            else:
+                gs = g_sorted_w.contiguous()
+                grad_w = torch.empty(T * k, dtype=gs.dtype, device=gs.device)
+                with _on_device(gs.device), _span("permute_gate_grad"):
+                    rc = _abi.lib().fmoe_permute_gate_grad(
+                        slot_pos.data_ptr(), T * k, gs.data_ptr(), _FLOAT_CODES[gs.dtype],
+                        grad_w.data_ptr(), _stream_handle(gs.device))
+                _abi.check(rc, "fmoe_permute_gate_grad")
+        if grad_w is not None:
             grad_w = grad_w.view(T, k)
         return grad_x, grad_w, None, None, None
 

@@ -375,6 +375,20 @@ FMOE_API int fmoe_permute_gather(const int32_t* d_slot_pos, int64_t num_tokens, 
 FMOE_API int fmoe_permute_gate_grad(const int32_t* d_slot_pos, int64_t num_slots,
                            const void* d_grad_sorted, int dtype, void* d_grad_gates, void* stream);
 
+/*
+ * Both gradients of the permutation in one launch, for top_k <= 64 (they replace the backward of
+ * tiny_model.py:133 and :128):
+ *   grad_x[t, :]  = the sum of grad_rows[d_slot_pos[t * top_k + j], :] over j, in ascending
+ *                   packed-row order, in fp32, rounded once (what fmoe_build_plan_from_slots +
+ *                   fmoe_combine_fwd with unit gates give, bit for bit)
+ *   grad_gates[i] = grad_sorted[d_slot_pos[i]]  (d_grad_sorted and d_grad_gates NULL: skipped)
+ * grad_rows [T * top_k, hidden] and grad_x [T, hidden] are contiguous, of `dtype`.
+ */
+FMOE_API int fmoe_permute_backward(const int32_t* d_slot_pos, int64_t num_tokens, int64_t top_k,
+                          int64_t hidden, int dtype, const void* d_grad_rows, void* d_grad_x,
+                          const void* d_grad_sorted, int gate_dtype, void* d_grad_gates,
+                          void* stream);
+
 #ifdef __cplusplus
 }
 #endif
