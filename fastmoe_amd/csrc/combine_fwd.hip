@@ -49,6 +49,10 @@ __device__ __forceinline__ void add_rows(const LaneRecs& lr, int cnt, uint32_t x
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
+      // Used whether or not the row exists, so that the compiler does not move the row's loads
+      // into the branch below, behind the other rows'.
+#pragma unroll
+      for (int u = 0; u < U; ++u) asm volatile("" : "+v"(a[r][u]));
       if (i + r < cnt) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -589,6 +593,7 @@ struct FwdArgs {
   void* out;
   int64_t out_stride;
   int accumulate;
+  unsigned lds;  // dynamic LDS of the deterministic kernel (DetTile)
   hipStream_t s;
 };
 
@@ -617,7 +622,7 @@ static int launch_fwd_k(const FwdArgs& a, int64_t chunks) {
     if (int rc = grid_for(a.T * chunks, "fmoe_combine_fwd(det)", &blocks)) return rc;
     const int persist = (int)fmoe_host::opt(fmoe_host::kOptFwdGrid);  // 0 = one wave per unit
     if (persist > 0 && (unsigned)persist < blocks) blocks = (unsigned)persist;
-    hipLaunchKernelGGL((k_fwd_det<TX, TO, V, U, RB>), dim3(blocks), dim3(kGroup), 0, a.s, a.status,
+    hipLaunchKernelGGL((k_fwd_det<TX, TO, V, U, RB>), dim3(blocks), dim3(kGroup), a.lds, a.s, a.status,
                        a.row_ptr, a.rec, static_cast<TO*>(a.out), a.out_stride, (uint32_t)a.D,
                        (uint32_t)a.T, (uint32_t)chunks, a.accumulate,
                        !a.accumulate && a.T * a.D * (int64_t)sizeof(TO) >= kOutStreamBytes);
@@ -654,34 +659,67 @@ static int launch_fwd_u(const FwdArgs& a) {
   return launch_fwd_k<TX, TO, V, U, RB>(a, chunks);
 }
 
-// Tile of the deterministic forward by the average rows per token r = N / T.  A batch issues its
-// R x U loads whether or not its rows exist (the spare slots read an empty range: no traffic, but
-// an issue slot each), so short segments take short batches: r <= 1.5 takes R = 2 (U = 4, with a
-// partly empty last chunk if D needs it, when D holds one chunk of 4 vectors per lane), r <= 3
-// takes R = 4.  Long segments (r >= 7) whose chunk
-// would be 2 vectors per lane take 1 with R = 8.  Measured with HIP events on one MI355X, bf16,
-// against the choice by D alone: T=16384, D=7168: k=1 129 -> 75 us, k=2 146 -> 109 us, k=8 355 ->
-// 349 us (Zipf) and 361 -> 354 us (top-k); D=5120, 3072, 6144 at k=8 about 2 % faster; D=4096 and
-// 16384 at k=2, 6 and 8 unchanged.
-static void pick_det_tile(int64_t N, int64_t T, int64_t D, int V, int* U, int* R) {
-  *U = pick_u(D, V);
-  *R = *U >= 4 ? 4 : 8;
-  if (fmoe_host::opt(fmoe_host::kOptFwdDetU) != 0 || N == 0) return;  // U forced: keep R by U
-  if (2 * N <= 3 * T && D >= (int64_t)kWave * V * 4) {  // r <= 1.5, a whole chunk of 4
-    *U = 4;
-    *R = 2;
-  } else if (N <= 3 * T) {                              // r <= 3
-    if (*U >= 2) *R = 4;
-  } else if (N >= 7 * T && *U == 2) {                   // r >= 7
-    *U = 1;
-    *R = 8;
+// Tile of the deterministic forward: U vectors per lane per row, R rows per batch, and `lds` bytes
+// of unused dynamic LDS, which bound the workgroups resident on a CU.
+struct DetTile {
+  int U, R;
+  unsigned lds;
+};
+// The most LDS that still lets `groups` workgroups share a CU's 160 KB, which is handed out in
+// pieces of 1280 bytes.
+constexpr unsigned lds_for_groups(int groups) { return (160u << 10) / 1280 / groups * 1280; }
+
+// The choice by the rows per token r = N / T and the bytes of the rows.
+//
+// Short segments.  A batch issues its R x U loads whether or not its rows exist (the spare slots
+// read an empty range: no traffic, but an issue slot each), so r <= 1.5 takes R = 2 (U = 4, with a
+// partly empty last chunk if D needs it, when D holds one chunk of 4 vectors per lane) and r < 2.5
+// takes R = 4.  bf16, T=16384, D=7168, us against the choice by D alone: k=1 129 -> 75, k=2 146 ->
+// 109.
+//
+// Longer segments are bound by how HBM serves thousands of row pieces read side by side, and lose
+// rate when more of them are in flight than its latency needs (64 to 96 KB of loads per CU).  Rows
+// that the 256 MB Infinity Cache cannot hold therefore take U = 2, R = 4 with 4 resident workgroups
+// per CU for r < 3.5, 3 beyond, and 2 for r >= 7 from 768 MB; smaller ones, which finish in a few
+// rounds, take U = 4, R = 2 with every slot in use.  bf16 (three sets of buffers in turn, us, the
+// previous choice -> this one; the same tile without the bound in brackets):
+//   T=4096, D=16384, k=8   208.2 -> 198.5 (212.8)     T=8192, D=16384, k=6   325.0 -> 308.8 (346.2)
+//   T=16384, D=7168, k=8   374.4 -> 348.8 (379.2)     T=8192, D=16384, k=5   272.0 -> 260.9 (286.3)
+//   T=16384, D=4096, k=8   211.2 -> 199.9 (214.8)     T=16384, D=16384, k=4  461.5 -> 429.1 (466.5)
+//   T=8192, D=4096, k=6     76.5 ->  75.6 ( 76.9)     T=16384, D=7168, k=3   157.4 -> 149.1 (157.5)
+//   T=4096, D=8192, k=8     99.6 ->  96.7 ( 99.6)     T=8192, D=3072, k=8     75.7 ->  73.7 ( 75.7)
+//   T=1024, D=7168, k=8     25.2 ->  23.4             T=512, D=7168, k=8      13.3 ->  11.9
+//   fp32: T=4096, D=16384, k=8  427.4 -> 404.0 (433.4); k=4  227.7 -> 215.7 (224.9)
+// With 2 workgroups T=8192, D=4096, k=6 takes 81.7 us and T=4096, D=8192, k=8 98.1; r < 2.5 loses
+// under every bound (T=8192, D=4096, k=2: 31.9, 36.7 with 3 workgroups).
+static DetTile pick_det_tile(int64_t N, int64_t T, int64_t D, int64_t x_bytes, int V) {
+  DetTile c{pick_u(D, V), 0, 0};
+  c.R = c.U >= 4 ? 4 : 8;
+  if (fmoe_host::opt(fmoe_host::kOptFwdDetU) != 0 || N == 0) return c;  // U forced: keep R by U
+  const int64_t bytes = N * D * x_bytes;
+  if (2 * N <= 3 * T && D >= (int64_t)kWave * V * 4) return {4, 2, 0};  // r <= 1.5
+  if (2 * N < 5 * T) {                                                  // r < 2.5
+    if (c.U >= 2) c.R = 4;
+    return c;
   }
+  if (D < (int64_t)kWave * V * 2) return c;  // less than a chunk of 2 vectors per lane
+  if (bytes >= (int64_t(256) << 20)) {
+    if (2 * N < 7 * T) return {2, 4, lds_for_groups(4)};
+    if (N >= 7 * T && bytes >= (int64_t(768) << 20)) return {2, 4, lds_for_groups(2)};
+    return {2, 4, lds_for_groups(3)};
+  }
+  if (2 * N < 7 * T) {  // 2.5 <= r < 3.5
+    if (c.U >= 2) c.R = 4;
+    return c;
+  }
+  if (D >= (int64_t)kWave * V * 4) return {4, 2, 0};
+  return {2, 4, 0};
 }
 
 // Tile shapes (U vectors per lane per row, R rows per batch).  The "fwd_tile" option <U><R> (e.g.
 // 44) overrides the choice for tuning.
 template <typename TX, typename TO, int V>
-static int launch_fwd_v(const FwdArgs& a) {
+static int launch_fwd_v(FwdArgs a) {
   if constexpr (V == 1) {
     return launch_fwd_u<TX, TO, 1, 4, 4>(a);
   } else {
@@ -691,7 +729,10 @@ static int launch_fwd_v(const FwdArgs& a) {
     if (!((U == 4 && (R == 4 || R == 2)) || (U == 2 && (R == 8 || R == 4)) ||
           (U == 1 && R == 8))) {
       if (a.mode == FMOE_MODE_DET) {
-        pick_det_tile(a.N, a.T, a.D, V, &U, &R);
+        const DetTile c = pick_det_tile(a.N, a.T, a.D, sizeof(TX), V);
+        U = c.U;
+        R = c.R;
+        a.lds = c.lds;
       } else {
         U = pick_u(a.D, V);
         R = U >= 4 ? 4 : 8;
@@ -737,6 +778,7 @@ struct SlotsBwdArgs {
   const void* gates;
   void* grad_gates;
   hipStream_t s;
+  unsigned lds;  // DetTile
 };
 
 template <typename TX, int V, int U, int RB, bool GATES, typename TG>
@@ -745,7 +787,7 @@ static int launch_slots_bwd_k(const SlotsBwdArgs& a) {
   const int64_t chunks = (a.D + CW - 1) / CW;
   unsigned blocks;
   if (int rc = grid_for(a.T * chunks, "fmoe_permute_backward", &blocks)) return rc;
-  hipLaunchKernelGGL((k_slots_bwd<TX, V, U, RB, GATES, TG>), dim3(blocks), dim3(kGroup), 0, a.s,
+  hipLaunchKernelGGL((k_slots_bwd<TX, V, U, RB, GATES, TG>), dim3(blocks), dim3(kGroup), a.lds, a.s,
                      a.slot_pos, (uint32_t)a.k, (uint32_t)(a.T * a.k),
                      static_cast<const TX*>(a.rows), (uint32_t)a.D, (uint32_t)a.T,
                      (uint32_t)chunks, static_cast<TX*>(a.out),
@@ -764,17 +806,17 @@ static int launch_slots_bwd_g(const SlotsBwdArgs& a, int gate_dtype) {
 
 // 16-byte vectors when every row is 16-byte aligned, else one element per lane.
 template <typename TX>
-static int launch_slots_bwd(const SlotsBwdArgs& a, int gate_dtype) {
+static int launch_slots_bwd(SlotsBwdArgs a, int gate_dtype) {
   constexpr int V = vec16<TX>();
   const bool vec_ok = a.D % V == 0 && (uintptr_t)a.rows % 16 == 0 && (uintptr_t)a.out % 16 == 0 &&
                       fmoe_host::opt(fmoe_host::kOptForceScalar) == 0;
   if (!vec_ok) return launch_slots_bwd_g<TX, 1, 4, 4>(a, gate_dtype);
-  int U, R;
-  pick_det_tile(a.T * a.k, a.T, a.D, V, &U, &R);
-  if (U == 4 && R == 2) return launch_slots_bwd_g<TX, V, 4, 2>(a, gate_dtype);
-  if (U == 4) return launch_slots_bwd_g<TX, V, 4, 4>(a, gate_dtype);
-  if (U == 2 && R == 4) return launch_slots_bwd_g<TX, V, 2, 4>(a, gate_dtype);
-  if (U == 2) return launch_slots_bwd_g<TX, V, 2, 8>(a, gate_dtype);
+  const DetTile c = pick_det_tile(a.T * a.k, a.T, a.D, sizeof(TX), V);
+  a.lds = c.lds;
+  if (c.U == 4 && c.R == 2) return launch_slots_bwd_g<TX, V, 4, 2>(a, gate_dtype);
+  if (c.U == 4) return launch_slots_bwd_g<TX, V, 4, 4>(a, gate_dtype);
+  if (c.U == 2 && c.R == 4) return launch_slots_bwd_g<TX, V, 2, 4>(a, gate_dtype);
+  if (c.U == 2) return launch_slots_bwd_g<TX, V, 2, 8>(a, gate_dtype);
   return launch_slots_bwd_g<TX, V, 1, 8>(a, gate_dtype);
 }
 
@@ -1033,7 +1075,7 @@ extern "C" int fmoe_permute_backward(const int32_t* d_slot_pos, int64_t num_toke
   FMOE_REQUIRE(!d_grad_gates || fmoe_host::is_float_dtype(gate_dtype),
                "fmoe_permute_backward: bad gate dtype %d", gate_dtype);
   const SlotsBwdArgs a{d_slot_pos, T, K, D, d_grad_rows, d_grad_x, d_grad_sorted, d_grad_gates,
-                       static_cast<hipStream_t>(stream)};
+                       static_cast<hipStream_t>(stream), 0};
   switch (dtype) {
     case FMOE_F32: return launch_slots_bwd<float>(a, gate_dtype);
     case FMOE_BF16: return launch_slots_bwd<bf16_t>(a, gate_dtype);
