@@ -155,7 +155,7 @@ __global__ __launch_bounds__(kGroup) void k_fwd_det(const int32_t* __restrict__ 
 // moves the token's gate gradients.  A slot_pos entry outside [0, N) adds nothing.
 // Bound by HBM like k_fwd_det.  T=8192, D=4096, top-6, bf16, permutation and its backward: 195.6 us
 // with the slot-map plan, the combine and the gate-gradient kernel (and autograd's fills of the
-// integer outputs' gradients), 184.4 us with this kernel alone.
+// integer outputs' gradients), 184.4 us with this kernel alone and k_fwd_det's tiles of then.
 template <typename TX, int V, int U, int RB, bool GATES, typename TG>
 __global__ __launch_bounds__(kGroup) void k_slots_bwd(const int32_t* __restrict__ slot_pos,
                                                       uint32_t k, uint32_t N,
@@ -781,6 +781,13 @@ struct SlotsBwdArgs {
   unsigned lds;  // DetTile
 };
 
+// grad_x is streamed from a smaller size than the forward's output (kOutStreamBytes): a backward is
+// always followed by more passes over as much data, which pay for the lines left in the cache.
+// Permutation forward + backward, three sets of buffers in turn, bf16, temporal / non-temporal:
+// T=8192, D=4096, top-6 and T=4096, D=8192, top-6 (64 MiB) 180.9 / 165.9 and 182.0 / 164.8 us;
+// 28 and 32 MiB of grad_x make no difference.
+constexpr int64_t kSlotsStreamBytes = int64_t(48) << 20;
+
 template <typename TX, int V, int U, int RB, bool GATES, typename TG>
 static int launch_slots_bwd_k(const SlotsBwdArgs& a) {
   const int64_t CW = (int64_t)kWave * V * U;
@@ -791,7 +798,7 @@ static int launch_slots_bwd_k(const SlotsBwdArgs& a) {
                      a.slot_pos, (uint32_t)a.k, (uint32_t)(a.T * a.k),
                      static_cast<const TX*>(a.rows), (uint32_t)a.D, (uint32_t)a.T,
                      (uint32_t)chunks, static_cast<TX*>(a.out),
-                     a.T * a.D * (int64_t)sizeof(TX) >= kOutStreamBytes,
+                     a.T * a.D * (int64_t)sizeof(TX) >= kSlotsStreamBytes,
                      static_cast<const TG*>(a.gates), static_cast<TG*>(a.grad_gates));
   return fmoe_host::check_launch("fmoe_permute_backward");
 }
