@@ -98,6 +98,12 @@ SIGNATURES: dict[str, tuple] = {
         _c_int,
         [_c_vp, _c_i64, _c_i64, _c_i64, _c_int, _c_vp, _c_vp, _c_vp, _c_int, _c_vp, _c_vp],
     ),
+    "fmoe_permute_small_max_slots": (_c_i64, []),
+    "fmoe_permute": (
+        _c_int,
+        [_c_vp, _c_int, _c_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_vp, _c_vp,
+         _c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp],
+    ),
 }
 
 _LIB: ctypes.CDLL | None = None

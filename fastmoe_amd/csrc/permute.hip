@@ -8,7 +8,8 @@
 // torch.argsort(..., stable=True) gives; the reference's unstable argsort (:112) leaves the order
 // of equal ids unspecified.
 //
-// Slot i = t * k + j is token t's j-th routing choice.  Steps (caller's stream, no host sync):
+// Slot i = t * k + j is token t's j-th routing choice.  Up to kPermSmallSlots slots, one launch does
+// all of it (k_perm_small).  Beyond, the steps are (caller's stream, no host sync):
 //   1. rank    one workgroup per block of 1024 slots (256 when E > 1024): each slot's stable rank among the
 //              block's slots of the same expert (wave ballots on the key bits give the lanes of
 //              a wave with an equal key; per-wave counts in LDS give the waves before it), and
@@ -17,6 +18,7 @@
 //              through LDS tiles), then the exclusive prefix over experts of the totals -> offsets.
 //   3. fill    one thread per slot: pos = off[e] + blkcnt[b][e] + rank; writes the reverse map,
 //              the gate in packed order and the slot -> row map (slot_pos).
+//      Up to kPermPlaceBlocks ranking blocks one kernel does 2 and 3 (k_perm_place).
 //   4. gather  one workgroup per token: its waves copy x[t] into the token's k packed rows (the row
 //              is read once from HBM and shared through L2; the copies are streaming stores).
 // An expert id outside [0, E) is key E: such slots go to the tail, after every expert's rows, and
@@ -24,7 +26,7 @@
 #include <algorithm>
 #include <cstdlib>
 
-#include "common.h"
+#include "plan.h"
 
 namespace fmoe {
 
@@ -228,14 +230,167 @@ __global__ __launch_bounds__(kGroup) void k_perm_fill(const TI* __restrict__ ids
   slot_pos[i] = pos;
 }
 
+// Steps 2 and 3 in one launch: a workgroup per ranking block b (1024 slots).  Thread e sums column e
+// of the block-count table -- the rows before b give the block's first place in expert e, all of
+// them the expert's total -- and the workgroup scans the totals into the offsets, so no workgroup
+// waits for another and the table is not rewritten.  Every workgroup reads the whole table (nb *
+// (E + 1) * 4 bytes, from L2), one thread per column, so its time grows with nb whatever E, while
+// the scan's grows with both: it is taken up to 64 blocks, and up to 256 from 128 experts.  The
+// build in us, rank + scan + fill -> rank + place (one MI355X, launches queued back to back):
+//   N=49152, E=64    10.9 -> 8.8     N=131072, E=256   19.7 -> 14.1    N=65536, E=1023  23.5 -> 12.3
+//   N=65536, E=16    10.7 -> 9.1     N=262144, E=1023  65.3 -> 27.3
+// (N=262144, E=8, which keeps the scan, took 20.1 against 15.9.)
+constexpr int kPermPlaceBlocks = 256;
+static bool place_blocks(int64_t nb, int64_t E) {
+  return nb <= 64 || (nb <= kPermPlaceBlocks && E >= 128);
+}
+template <typename TI, typename TG>
+__global__ __launch_bounds__(kPermBlockLarge) void k_perm_place(
+    const TI* __restrict__ ids, const TG* __restrict__ gates, int64_t N, int64_t E, int64_t k,
+    int nb, const int32_t* __restrict__ blkcnt, const int32_t* __restrict__ rank,
+    int64_t* __restrict__ counts, int64_t* __restrict__ offsets, int64_t* __restrict__ rev,
+    TG* __restrict__ sorted_gates, int32_t* __restrict__ slot_pos, int32_t* __restrict__ status) {
+  static_assert(kPermBlockLarge == kScanThreads, "block_exclusive_scan_1024");
+  __shared__ int32_t first[kPermSmallExperts + 1];
+  const int E1 = (int)E + 1;
+  const int b = (int)blockIdx.x;
+  const int64_t i = (int64_t)b * kPermBlockLarge + threadIdx.x;
+  const bool live = i < N;
+  const int key = live ? slot_key(ids, i, E) : 0;
+  const int in_block = live ? rank[i] : 0;
+  int carry = 0;
+  for (int k0 = 0; k0 < E1; k0 += kScanThreads) {  // twice at most (E = 1024)
+    const int e = k0 + (int)threadIdx.x;
+    int total = 0, before = 0;
+    if (e < E1) {
+      constexpr int kRows = 16;  // independent loads in flight
+      for (int r0 = 0; r0 < nb; r0 += kRows) {
+        int c[kRows];
+#pragma unroll
+        for (int r = 0; r < kRows; ++r)
+          c[r] = r0 + r < nb ? blkcnt[(int64_t)(r0 + r) * E1 + e] : 0;
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+          total += c[r];
+          before += r0 + r < b ? c[r] : 0;
+        }
+      }
+    }
+    int all;
+    const int excl = carry + block_exclusive_scan_1024(total, &all);
+    if (e < E1) {
+      first[e] = excl + before;
+      if (b == 0) {
+        if (e < (int)E) {
+          counts[e] = total;
+          offsets[e] = excl;
+        } else {
+          offsets[E] = excl;   // rows of valid slots
+          status[0] = total;   // slots with an id outside [0, E)
+        }
+      }
+    }
+    carry += all;
+  }
+  __syncthreads();
+  if (live) {
+    const int pos = first[key] + in_block;
+    rev[pos] = i / k;
+    sorted_gates[pos] = gates[i];
+    slot_pos[i] = pos;
+  }
+}
+
+// Row copy, VB bytes per lane access, by one wave: cached reads (the token's other rows read the
+// same bytes), non-temporal stores.
+template <int VB>
+__device__ __forceinline__ void copy_row(rsrc_t rs, rsrc_t rd, uint32_t row_bytes, int lane) {
+  constexpr int U = VB == 16 ? 8 : 4;  // accesses in flight per lane
+  using R = Raw<VB>;
+  using raw_t = typename R::type;
+  for (uint32_t base = 0; base < row_bytes; base += (uint32_t)(kWave * VB * U)) {
+    raw_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      v[u] = R::template ld<kCPolCached>(rs, base + (uint32_t)(u * kWave + lane) * VB);
+#pragma unroll
+    for (int u = 0; u < U; ++u)  // bytes past the row: dropped by the range check
+      R::template st<kCPol>(rd, base + (uint32_t)(u * kWave + lane) * VB, v[u]);
+  }
+}
+
+// ---- small inputs: the whole permutation in one launch ---------------------------------------
+// A decoding step's permutation is four dependent launches of about 4 us each around microseconds
+// of work.  Here every workgroup stages all N keys in LDS as (key << 16 | slot), distinct values
+// whose order is the packed order, so a slot's packed row is the number of smaller values: a wave
+// counts them for its slot (N / 64 compares per lane), writes the slot's outputs and copies its
+// row.  Expert e's first row is the number of values below e << 16; those E + 1 counts are spread
+// over the waves of the grid.  Staging reads the N ids once per workgroup from L2, so the gain over
+// rank + place + gather shrinks with N (one MI355X, top-8, E=256, D=7168, bf16, us): N=128 14.1 ->
+// 8.1, N=1024 14.4 -> 9.1, N=2048 16.7 -> 11.1, N=4096 22.4 -> 17.4, where the rows' own copy is
+// most of it.
+constexpr int kPermSmallSlots = 4096;
+constexpr int kPermSmallWaves = 8;
+constexpr unsigned kPermSmallGroups = 1024;
+static_assert(kPermMaxExperts < (1 << 15) && kPermSmallSlots <= (1 << 16), "32-bit sort values");
+
+// Number of values below `lim` among v[0 .. n4 * 4), counted by one wave (every lane gets it).
+__device__ __forceinline__ int count_below(const u32x4* v, int n4, uint32_t lim, int lane) {
+  int c = 0;
+  for (int q = lane; q < n4; q += kWave) {
+    const u32x4 x = v[q];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) c += x[r] < lim ? 1 : 0;
+  }
+  return __builtin_amdgcn_readlane(wave_incl_sum(c), kWave - 1);
+}
+
+template <typename TI, typename TG, int VB>
+__global__ __launch_bounds__(kPermSmallWaves * kWave) void k_perm_small(
+    const TI* __restrict__ ids, const TG* __restrict__ gates, uint32_t N, uint32_t k, uint32_t E,
+    const uint8_t* __restrict__ x, int64_t x_stride_bytes, uint8_t* __restrict__ out,
+    uint32_t row_bytes, int64_t* __restrict__ counts, int64_t* __restrict__ offsets,
+    int64_t* __restrict__ rev, TG* __restrict__ sorted_gates, int32_t* __restrict__ slot_pos,
+    int32_t* __restrict__ status) {
+  __shared__ __attribute__((aligned(16))) uint32_t val[kPermSmallSlots];
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint32_t wave = (uint32_t)uniform(threadIdx.x / kWave);
+  const uint32_t padded = (N + 3) & ~3u;
+  for (uint32_t i = threadIdx.x; i < padded; i += kPermSmallWaves * kWave)
+    val[i] = i < N ? ((uint32_t)slot_key(ids, i, E) << 16) | i : 0xffffffffu;
+  __syncthreads();
+  const u32x4* v = reinterpret_cast<const u32x4*>(val);
+  const int n4 = (int)(padded / 4);
+  const uint32_t first = blockIdx.x * kPermSmallWaves + wave;
+  const uint32_t waves = gridDim.x * kPermSmallWaves;
+  for (uint32_t i = first; i < N; i += waves) {
+    const uint32_t pos = (uint32_t)count_below(v, n4, val[i], lane);
+    const uint32_t t = i / k;
+    if (lane == 0) {
+      rev[pos] = t;
+      sorted_gates[pos] = gates[i];
+      slot_pos[i] = (int32_t)pos;
+    }
+    if (row_bytes)  // wave-uniform
+      copy_row<VB>(make_rsrc(x + (int64_t)t * x_stride_bytes, row_bytes),
+                   make_rsrc(out + (int64_t)pos * row_bytes, row_bytes), row_bytes, lane);
+  }
+  for (uint32_t e = first; e <= E; e += waves) {
+    const int lo = count_below(v, n4, e << 16, lane);
+    const int hi = e < E ? count_below(v, n4, (e + 1) << 16, lane) : (int)N;
+    if (lane == 0) {
+      offsets[e] = lo;
+      if (e < E) counts[e] = hi - lo;
+      else status[0] = hi - lo;  // slots with an id outside [0, E)
+    }
+  }
+}
+
 // Row copy x[t] -> out[slot_pos[t * k + j]] for j < k, VB bytes per lane access.
 template <int VB>
 __global__ __launch_bounds__(kPermGatherWaves * kWave) void k_perm_gather(
     const int32_t* __restrict__ slot_pos, int64_t k, const uint8_t* __restrict__ x,
     int64_t x_stride_bytes, uint8_t* __restrict__ out, uint32_t row_bytes, int64_t N) {
-  constexpr int U = VB == 16 ? 8 : 4;  // accesses in flight per lane
-  using R = Raw<VB>;
-  using raw_t = typename R::type;
   const int64_t t = blockIdx.x;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = uniform(threadIdx.x / kWave);
@@ -243,16 +398,7 @@ __global__ __launch_bounds__(kPermGatherWaves * kWave) void k_perm_gather(
   for (int64_t j = wave; j < k; j += kPermGatherWaves) {
     const int64_t pos = slot_pos[t * k + j];
     if (pos < 0 || pos >= N) continue;  // slot_pos comes from fmoe_permute_build: always in range
-    const rsrc_t rd = make_rsrc(out + pos * (int64_t)row_bytes, row_bytes);
-    for (uint32_t base = 0; base < row_bytes; base += (uint32_t)(kWave * VB * U)) {
-      raw_t v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        v[u] = R::template ld<kCPolCached>(rs, base + (uint32_t)(u * kWave + lane) * VB);
-#pragma unroll
-      for (int u = 0; u < U; ++u)  // bytes past the row: dropped by the range check
-        R::template st<kCPol>(rd, base + (uint32_t)(u * kWave + lane) * VB, v[u]);
-    }
+    copy_row<VB>(rs, make_rsrc(out + pos * (int64_t)row_bytes, row_bytes), row_bytes, lane);
   }
 }
 
@@ -271,45 +417,47 @@ __global__ __launch_bounds__(kGroup) void k_perm_gate_grad(const int32_t* __rest
 
 using namespace fmoe;
 
+// Bytes per lane access of a row copy: 16, 4 or 2, as the rows' lengths and addresses allow.
+static int row_align(int64_t row_bytes, const void* x, const void* out, int64_t x_stride) {
+  const uint64_t all = (uint64_t)row_bytes | (uintptr_t)x | (uintptr_t)out | (uint64_t)x_stride;
+  return all % 16 == 0 ? 16 : (all % 4 == 0 ? 4 : 2);
+}
+
 extern "C" int64_t fmoe_permute_workspace_bytes(int64_t num_slots, int64_t num_experts) {
   if (num_slots < 0 || num_experts < 1) return -1;
   return perm_layout(num_slots, num_experts).total;
 }
 
-extern "C" int fmoe_permute_build(const void* d_expert_ids, int id_dtype, const void* d_gates,
-                                  int gate_dtype, int64_t num_tokens, int64_t top_k,
-                                  int64_t num_experts, int64_t* d_counts, int64_t* d_offsets,
-                                  int64_t* d_rev, void* d_sorted_gates, int32_t* d_slot_pos,
-                                  int32_t* d_status, void* d_workspace, void* stream) {
-  fmoe_host::clear_error();
+static int permute_build(const char* who, const void* d_expert_ids, int id_dtype,
+                         const void* d_gates, int gate_dtype, int64_t num_tokens, int64_t top_k,
+                         int64_t num_experts, int64_t* d_counts, int64_t* d_offsets,
+                         int64_t* d_rev, void* d_sorted_gates, int32_t* d_slot_pos,
+                         int32_t* d_status, void* d_workspace, hipStream_t s) {
   const int64_t T = num_tokens, K = top_k, E = num_experts;
-  FMOE_REQUIRE(T >= 0 && K >= 1, "fmoe_permute_build: bad sizes T=%lld k=%lld", (long long)T,
+  FMOE_REQUIRE(T >= 0 && K >= 1, "%s: bad sizes T=%lld k=%lld", who, (long long)T,
                (long long)K);
   FMOE_REQUIRE(E >= 1 && E <= kPermMaxExperts,
-               "fmoe_permute_build: num_experts %lld not in [1, %d]", (long long)E,
-               kPermMaxExperts);
+               "%s: num_experts %lld not in [1, %d]", who, (long long)E, kPermMaxExperts);
   if (K >= (int64_t(1) << 31) || (T > 0 && K > ((int64_t(1) << 31) - 1) / T)) {
-    fmoe_host::set_error("fmoe_permute_build: T*k exceeds the 32-bit row counters");
+    fmoe_host::set_error("%s: T*k exceeds the 32-bit row counters", who);
     return FMOE_ERANGE;
   }
   const int64_t N = T * K;
   const int blk = perm_block(E);
   const int64_t nb = (N + blk - 1) / blk;
   if (nb * (E + 1) >= (int64_t(1) << 31)) {
-    fmoe_host::set_error("fmoe_permute_build: block count table too large");
+    fmoe_host::set_error("%s: block count table too large", who);
     return FMOE_ERANGE;
   }
-  FMOE_REQUIRE(fmoe_host::is_index_dtype(id_dtype), "fmoe_permute_build: bad id dtype %d",
-               id_dtype);
-  FMOE_REQUIRE(fmoe_host::is_float_dtype(gate_dtype), "fmoe_permute_build: bad gate dtype %d",
+  FMOE_REQUIRE(fmoe_host::is_index_dtype(id_dtype), "%s: bad id dtype %d", who, id_dtype);
+  FMOE_REQUIRE(fmoe_host::is_float_dtype(gate_dtype), "%s: bad gate dtype %d", who,
                gate_dtype);
   FMOE_REQUIRE(d_counts && d_offsets && d_status && d_workspace,
-               "fmoe_permute_build: null device pointer");
+               "%s: null device pointer", who);
   FMOE_REQUIRE(N == 0 || (d_expert_ids && d_gates && d_rev && d_sorted_gates && d_slot_pos),
-               "fmoe_permute_build: null ids/gates/outputs");
+               "%s: null ids/gates/outputs", who);
   FMOE_REQUIRE(((uintptr_t)d_workspace & 255) == 0,
-               "fmoe_permute_build: workspace not 256B-aligned");
-  hipStream_t s = static_cast<hipStream_t>(stream);
+               "%s: workspace not 256B-aligned", who);
   const PermLayout L = perm_layout(N, E);
   char* ws = static_cast<char*>(d_workspace);
   int32_t* blkcnt = reinterpret_cast<int32_t*>(ws + L.blkcnt);
@@ -329,14 +477,30 @@ extern "C" int fmoe_permute_build(const void* d_expert_ids, int id_dtype, const 
       else FMOE_PRANK(int32_t, kPermMaxExperts, kPermBlockSmall);
     }
 #undef FMOE_PRANK
-    if (int rc = fmoe_host::check_launch("fmoe_permute_build(rank)")) return rc;
+    if (int rc = fmoe_host::check_launch(who)) return rc;
+  }
+  const bool g4 = fmoe_host::dtype_bytes(gate_dtype) == 4;
+  if (N > 0 && blk == kPermBlockLarge && place_blocks(nb, E)) {
+#define FMOE_PPLACE(TI, TG)                                                                        \
+  hipLaunchKernelGGL((k_perm_place<TI, TG>), dim3((unsigned)nb), dim3(kPermBlockLarge), 0, s,      \
+                     static_cast<const TI*>(d_expert_ids), static_cast<const TG*>(d_gates), N, E,  \
+                     K, (int)nb, blkcnt, rank, d_counts, d_offsets, d_rev,                         \
+                     static_cast<TG*>(d_sorted_gates), d_slot_pos, d_status)
+    if (id_dtype == FMOE_I64) {
+      if (g4) FMOE_PPLACE(int64_t, uint32_t);
+      else FMOE_PPLACE(int64_t, uint16_t);
+    } else {
+      if (g4) FMOE_PPLACE(int32_t, uint32_t);
+      else FMOE_PPLACE(int32_t, uint16_t);
+    }
+#undef FMOE_PPLACE
+    return fmoe_host::check_launch(who);
   }
   hipLaunchKernelGGL(k_perm_scan, dim3(1), dim3(kPermScanThreads), 0, s, blkcnt, nb, E, off,
                      d_counts, d_offsets, d_status);
-  if (int rc = fmoe_host::check_launch("fmoe_permute_build(scan)")) return rc;
+  if (int rc = fmoe_host::check_launch(who)) return rc;
   if (N == 0) return FMOE_OK;
   const dim3 grid((unsigned)((N + kGroup - 1) / kGroup));
-  const bool g4 = fmoe_host::dtype_bytes(gate_dtype) == 4;
 #define FMOE_PFILL(TI, TG)                                                                         \
   hipLaunchKernelGGL((k_perm_fill<TI, TG>), grid, dim3(kGroup), 0, s,                              \
                      static_cast<const TI*>(d_expert_ids), static_cast<const TG*>(d_gates), N, E,  \
@@ -350,48 +514,138 @@ extern "C" int fmoe_permute_build(const void* d_expert_ids, int id_dtype, const 
     else FMOE_PFILL(int32_t, uint16_t);
   }
 #undef FMOE_PFILL
-  return fmoe_host::check_launch("fmoe_permute_build(fill)");
+  return fmoe_host::check_launch(who);
+}
+
+extern "C" int fmoe_permute_build(const void* d_expert_ids, int id_dtype, const void* d_gates,
+                                  int gate_dtype, int64_t num_tokens, int64_t top_k,
+                                  int64_t num_experts, int64_t* d_counts, int64_t* d_offsets,
+                                  int64_t* d_rev, void* d_sorted_gates, int32_t* d_slot_pos,
+                                  int32_t* d_status, void* d_workspace, void* stream) {
+  fmoe_host::clear_error();
+  return permute_build("fmoe_permute_build", d_expert_ids, id_dtype, d_gates, gate_dtype,
+                       num_tokens, top_k, num_experts, d_counts, d_offsets, d_rev, d_sorted_gates,
+                       d_slot_pos, d_status, d_workspace, static_cast<hipStream_t>(stream));
+}
+
+// The checks of fmoe_permute_gather's rows.
+static int check_rows(const char* who, int64_t T, int64_t K, int64_t row_bytes, const void* d_x,
+                      int64_t x_row_stride_bytes, const void* d_out) {
+  FMOE_REQUIRE(T >= 0 && K >= 1 && row_bytes >= 1, "%s: bad sizes T=%lld k=%lld row_bytes=%lld",
+               who, (long long)T, (long long)K, (long long)row_bytes);
+  if (row_bytes >= (int64_t(1) << 31) || T >= (int64_t(1) << 31) ||
+      (T > 0 && K > ((int64_t(1) << 31) - 1) / T)) {
+    fmoe_host::set_error("%s: sizes exceed the 32-bit row counters", who);
+    return FMOE_ERANGE;
+  }
+  if (T == 0) return FMOE_OK;
+  FMOE_REQUIRE(d_x && d_out, "%s: null device pointer", who);
+  FMOE_REQUIRE(x_row_stride_bytes >= row_bytes || T == 1,
+               "%s: x rows overlap (stride %lld < %lld bytes)", who,
+               (long long)x_row_stride_bytes, (long long)row_bytes);
+  FMOE_REQUIRE(row_bytes % 2 == 0 && (uintptr_t)d_x % 2 == 0 && (uintptr_t)d_out % 2 == 0 &&
+                   x_row_stride_bytes % 2 == 0,
+               "%s: rows must be 2-byte aligned", who);
+  return FMOE_OK;
+}
+
+static int launch_gather(const char* who, const int32_t* d_slot_pos, int64_t T, int64_t K,
+                         int64_t row_bytes, const void* d_x, int64_t x_row_stride_bytes,
+                         void* d_out, hipStream_t s) {
+  const int al = row_align(row_bytes, d_x, d_out, x_row_stride_bytes);
+  const dim3 grid((unsigned)T), block(kPermGatherWaves * kWave);
+  const uint8_t* x = static_cast<const uint8_t*>(d_x);
+  uint8_t* out = static_cast<uint8_t*>(d_out);
+  if (al == 16)
+    hipLaunchKernelGGL(k_perm_gather<16>, grid, block, 0, s, d_slot_pos, K, x, x_row_stride_bytes,
+                       out, (uint32_t)row_bytes, T * K);
+  else if (al == 4)
+    hipLaunchKernelGGL(k_perm_gather<4>, grid, block, 0, s, d_slot_pos, K, x, x_row_stride_bytes,
+                       out, (uint32_t)row_bytes, T * K);
+  else
+    hipLaunchKernelGGL(k_perm_gather<2>, grid, block, 0, s, d_slot_pos, K, x, x_row_stride_bytes,
+                       out, (uint32_t)row_bytes, T * K);
+  return fmoe_host::check_launch(who);
 }
 
 extern "C" int fmoe_permute_gather(const int32_t* d_slot_pos, int64_t num_tokens, int64_t top_k,
                                    int64_t row_bytes, const void* d_x, int64_t x_row_stride_bytes,
                                    void* d_out, void* stream) {
   fmoe_host::clear_error();
-  const int64_t T = num_tokens, K = top_k;
-  FMOE_REQUIRE(T >= 0 && K >= 1 && row_bytes >= 1,
-               "fmoe_permute_gather: bad sizes T=%lld k=%lld row_bytes=%lld", (long long)T,
-               (long long)K, (long long)row_bytes);
-  if (row_bytes >= (int64_t(1) << 31) || T >= (int64_t(1) << 31) ||
-      (T > 0 && K > ((int64_t(1) << 31) - 1) / T)) {
-    fmoe_host::set_error("fmoe_permute_gather: sizes exceed the 32-bit row counters");
-    return FMOE_ERANGE;
-  }
-  if (T == 0) return FMOE_OK;
-  FMOE_REQUIRE(d_slot_pos && d_x && d_out, "fmoe_permute_gather: null device pointer");
-  FMOE_REQUIRE(x_row_stride_bytes >= row_bytes || T == 1,
-               "fmoe_permute_gather: x rows overlap (stride %lld < %lld bytes)",
-               (long long)x_row_stride_bytes, (long long)row_bytes);
-  FMOE_REQUIRE(row_bytes % 2 == 0 && (uintptr_t)d_x % 2 == 0 && (uintptr_t)d_out % 2 == 0 &&
-                   x_row_stride_bytes % 2 == 0,
-               "fmoe_permute_gather: rows must be 2-byte aligned");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  auto aligned = [&](int a) {
-    return row_bytes % a == 0 && (uintptr_t)d_x % a == 0 && (uintptr_t)d_out % a == 0 &&
-           x_row_stride_bytes % a == 0;
+  const char* who = "fmoe_permute_gather";
+  if (int rc = check_rows(who, num_tokens, top_k, row_bytes, d_x, x_row_stride_bytes, d_out))
+    return rc;
+  if (num_tokens == 0) return FMOE_OK;
+  FMOE_REQUIRE(d_slot_pos, "%s: null device pointer", who);
+  return launch_gather(who, d_slot_pos, num_tokens, top_k, row_bytes, d_x, x_row_stride_bytes,
+                       d_out, static_cast<hipStream_t>(stream));
+}
+
+static int launch_small(const char* who, const void* d_expert_ids, int id_dtype,
+                        const void* d_gates, int gate_dtype, int64_t T, int64_t K, int64_t E,
+                        int64_t row_bytes, const void* d_x, int64_t x_row_stride_bytes,
+                        int64_t* d_counts, int64_t* d_offsets, int64_t* d_rev,
+                        void* d_sorted_gates, int32_t* d_slot_pos, int32_t* d_status, void* d_out,
+                        hipStream_t s) {
+  const int64_t N = T * K;
+  const dim3 grid(std::min<unsigned>(kPermSmallGroups,
+                                     (unsigned)((N + kPermSmallWaves - 1) / kPermSmallWaves)));
+  auto launch = [&](auto ti, auto tg, auto vb) {
+    using TI = decltype(ti);
+    using TG = decltype(tg);
+    hipLaunchKernelGGL((k_perm_small<TI, TG, decltype(vb)::value>), grid,
+                       dim3(kPermSmallWaves * kWave), 0, s, static_cast<const TI*>(d_expert_ids),
+                       static_cast<const TG*>(d_gates), (uint32_t)N, (uint32_t)K, (uint32_t)E,
+                       static_cast<const uint8_t*>(d_x), x_row_stride_bytes,
+                       static_cast<uint8_t*>(d_out), (uint32_t)row_bytes, d_counts, d_offsets,
+                       d_rev, static_cast<TG*>(d_sorted_gates), d_slot_pos, d_status);
   };
-  const dim3 grid((unsigned)T), block(kPermGatherWaves * kWave);
-  const uint8_t* x = static_cast<const uint8_t*>(d_x);
-  uint8_t* out = static_cast<uint8_t*>(d_out);
-  if (aligned(16))
-    hipLaunchKernelGGL(k_perm_gather<16>, grid, block, 0, s, d_slot_pos, K, x, x_row_stride_bytes,
-                       out, (uint32_t)row_bytes, T * K);
-  else if (aligned(4))
-    hipLaunchKernelGGL(k_perm_gather<4>, grid, block, 0, s, d_slot_pos, K, x, x_row_stride_bytes,
-                       out, (uint32_t)row_bytes, T * K);
-  else
-    hipLaunchKernelGGL(k_perm_gather<2>, grid, block, 0, s, d_slot_pos, K, x, x_row_stride_bytes,
-                       out, (uint32_t)row_bytes, T * K);
-  return fmoe_host::check_launch("fmoe_permute_gather");
+  auto by_gate = [&](auto ti, auto vb) {
+    if (fmoe_host::dtype_bytes(gate_dtype) == 4) launch(ti, uint32_t{}, vb);
+    else launch(ti, uint16_t{}, vb);
+  };
+  auto by_id = [&](auto vb) {
+    if (id_dtype == FMOE_I64) by_gate(int64_t{}, vb);
+    else by_gate(int32_t{}, vb);
+  };
+  const int al = row_align(row_bytes, d_x, d_out, x_row_stride_bytes);
+  if (al == 16) by_id(std::integral_constant<int, 16>{});
+  else if (al == 4) by_id(std::integral_constant<int, 4>{});
+  else by_id(std::integral_constant<int, 2>{});
+  return fmoe_host::check_launch(who);
+}
+
+extern "C" int64_t fmoe_permute_small_max_slots(void) { return kPermSmallSlots; }
+
+extern "C" int fmoe_permute(const void* d_expert_ids, int id_dtype, const void* d_gates,
+                            int gate_dtype, int64_t num_tokens, int64_t top_k, int64_t num_experts,
+                            int64_t row_bytes, const void* d_x, int64_t x_row_stride_bytes,
+                            int64_t* d_counts, int64_t* d_offsets, int64_t* d_rev,
+                            void* d_sorted_gates, int32_t* d_slot_pos, int32_t* d_status,
+                            void* d_out, void* d_workspace, void* stream) {
+  fmoe_host::clear_error();
+  const char* who = "fmoe_permute";
+  const int64_t T = num_tokens, K = top_k, E = num_experts;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  FMOE_REQUIRE(T >= 1, "%s: bad sizes T=%lld k=%lld", who, (long long)T, (long long)K);
+  if (int rc = check_rows(who, T, K, row_bytes, d_x, x_row_stride_bytes, d_out)) return rc;
+  if (T * K <= kPermSmallSlots) {
+    FMOE_REQUIRE(E >= 1 && E <= kPermMaxExperts, "%s: num_experts %lld not in [1, %d]", who,
+                 (long long)E, kPermMaxExperts);
+    FMOE_REQUIRE(fmoe_host::is_index_dtype(id_dtype), "%s: bad id dtype %d", who, id_dtype);
+    FMOE_REQUIRE(fmoe_host::is_float_dtype(gate_dtype), "%s: bad gate dtype %d", who, gate_dtype);
+    FMOE_REQUIRE(d_expert_ids && d_gates && d_counts && d_offsets && d_rev && d_sorted_gates &&
+                     d_slot_pos && d_status,
+                 "%s: null device pointer", who);
+    return launch_small(who, d_expert_ids, id_dtype, d_gates, gate_dtype, T, K, E, row_bytes, d_x,
+                        x_row_stride_bytes, d_counts, d_offsets, d_rev, d_sorted_gates, d_slot_pos,
+                        d_status, d_out, s);
+  }
+  if (int rc = permute_build(who, d_expert_ids, id_dtype, d_gates, gate_dtype, T, K, E, d_counts,
+                             d_offsets, d_rev, d_sorted_gates, d_slot_pos, d_status, d_workspace,
+                             s))
+    return rc;
+  return launch_gather(who, d_slot_pos, T, K, row_bytes, d_x, x_row_stride_bytes, d_out, s);
 }
 
 extern "C" int fmoe_permute_gate_grad(const int32_t* d_slot_pos, int64_t num_slots,

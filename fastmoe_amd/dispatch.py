@@ -9,8 +9,9 @@ Mirrors the sort-and-gather half of ``MoEFeedForward.gate_and_sort``
     permuted_data       = x_flat[reverse_map_indices]                  (:133)
     expert_counts       = bincount(sorted expert ids, minlength=E)     (:138)
 
-computed by ``fmoe_permute_build`` (rank / scan / fill kernels) and ``fmoe_permute_gather`` (one
-workgroup per token copies its row into its k packed rows).  The packed order is the stable one:
+computed by ``fmoe_permute``: one launch for up to 4096 slots, beyond that ``fmoe_permute_build``
+(rank and place kernels) and ``fmoe_permute_gather`` (one workgroup per token copies its row into
+its k packed rows).  The packed order is the stable one:
 within an expert, slots keep ascending order.  The reference's argsort is unstable, so it leaves
 the order of equal ids unspecified; ``torch.argsort(..., stable=True)`` gives exactly this order.
 
@@ -28,7 +29,7 @@ from typing import NamedTuple, Optional
 
 import torch
 
-from . import _abi
+from . import _abi, ops
 from .ops import (_FLOAT_CODES, _INDEX_CODES, _launch_fwd, _on_device, _refuse_autograd_capture,
                   _require_cuda, _span, _stream_handle, _validate_default,
                   prepare_metadata_and_plan)
@@ -79,6 +80,16 @@ def _unit_gate_combine(rows: torch.Tensor, rev: torch.Tensor, num_tokens: int) -
     return out
 
 
+_SMALL_SLOTS: list = []
+
+
+def _small_slots() -> int:
+    """Slots up to which fmoe_permute is one launch and needs no workspace."""
+    if not _SMALL_SLOTS:
+        _SMALL_SLOTS.append(int(_abi.lib().fmoe_permute_small_max_slots()))
+    return _SMALL_SLOTS[0]
+
+
 class _TokenPermute(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x_flat, topk_weights, topk_indices, num_experts, validate):
@@ -96,25 +107,37 @@ class _TokenPermute(torch.autograd.Function):
         sorted_w = torch.empty(N, dtype=gates.dtype, device=dev)
         slot_pos = torch.empty(N, dtype=torch.int32, device=dev)
         status = torch.empty(1, dtype=torch.int32, device=dev)
-        nbytes = lib.fmoe_permute_workspace_bytes(N, E)
-        ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=dev)
-        out = torch.empty((N, D), dtype=x_flat.dtype, device=dev)
         es = x_flat.element_size()
+        out = torch.empty((N, D), dtype=x_flat.dtype, device=dev)
+        x_stride = (x_flat.stride(0) if T > 1 else D) * es
+        whole = N > 0 and D > 0 and ops._TIMER is None  # one call; timed: one per span
+        ws = None
+        if not whole or N > _small_slots():
+            ws = torch.empty(max(lib.fmoe_permute_workspace_bytes(N, E), 256), dtype=torch.uint8,
+                             device=dev)
         with _on_device(dev):
-            with _span("permute_build"):
-                rc = lib.fmoe_permute_build(
+            if whole:
+                rc = lib.fmoe_permute(
                     ids.data_ptr(), _INDEX_CODES[ids.dtype], gates.data_ptr(),
-                    _FLOAT_CODES[gates.dtype], T, k, E, counts.data_ptr(), offsets.data_ptr(),
-                    rev.data_ptr(), sorted_w.data_ptr(), slot_pos.data_ptr(), status.data_ptr(),
-                    ws.data_ptr(), _stream_handle(dev))
-            _abi.check(rc, "fmoe_permute_build")
-            if N and D:
-                with _span("permute_gather"):
-                    rc = lib.fmoe_permute_gather(
-                        slot_pos.data_ptr(), T, k, D * es, x_flat.data_ptr(),
-                        (x_flat.stride(0) if T > 1 else D) * es, out.data_ptr(),
-                        _stream_handle(dev))
-                _abi.check(rc, "fmoe_permute_gather")
+                    _FLOAT_CODES[gates.dtype], T, k, E, D * es, x_flat.data_ptr(), x_stride,
+                    counts.data_ptr(), offsets.data_ptr(), rev.data_ptr(), sorted_w.data_ptr(),
+                    slot_pos.data_ptr(), status.data_ptr(), out.data_ptr(),
+                    ws.data_ptr() if ws is not None else None, _stream_handle(dev))
+                _abi.check(rc, "fmoe_permute")
+            else:
+                with _span("permute_build"):
+                    rc = lib.fmoe_permute_build(
+                        ids.data_ptr(), _INDEX_CODES[ids.dtype], gates.data_ptr(),
+                        _FLOAT_CODES[gates.dtype], T, k, E, counts.data_ptr(), offsets.data_ptr(),
+                        rev.data_ptr(), sorted_w.data_ptr(), slot_pos.data_ptr(),
+                        status.data_ptr(), ws.data_ptr(), _stream_handle(dev))
+                _abi.check(rc, "fmoe_permute_build")
+                if N and D:
+                    with _span("permute_gather"):
+                        rc = lib.fmoe_permute_gather(
+                            slot_pos.data_ptr(), T, k, D * es, x_flat.data_ptr(), x_stride,
+                            out.data_ptr(), _stream_handle(dev))
+                    _abi.check(rc, "fmoe_permute_gather")
         if validate:
             bad = int(status[0])
             if bad:

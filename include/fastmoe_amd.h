@@ -389,6 +389,19 @@ FMOE_API int fmoe_permute_backward(const int32_t* d_slot_pos, int64_t num_tokens
                           const void* d_grad_sorted, int gate_dtype, void* d_grad_gates,
                           void* stream);
 
+/*
+ * fmoe_permute_build followed by fmoe_permute_gather on the same arguments, for T >= 1; outputs as
+ * in those two calls, bit for bit (d_out is packed [T * top_k, row_bytes]).  Up to
+ * fmoe_permute_small_max_slots() slots (4096) it is one launch and d_workspace may be NULL;
+ * beyond, the workspace is fmoe_permute_build's.
+ */
+FMOE_API int64_t fmoe_permute_small_max_slots(void);
+FMOE_API int fmoe_permute(const void* d_expert_ids, int id_dtype, const void* d_gates, int gate_dtype,
+                 int64_t num_tokens, int64_t top_k, int64_t num_experts, int64_t row_bytes,
+                 const void* d_x, int64_t x_row_stride_bytes, int64_t* d_counts,
+                 int64_t* d_offsets, int64_t* d_rev, void* d_sorted_gates, int32_t* d_slot_pos,
+                 int32_t* d_status, void* d_out, void* d_workspace, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
