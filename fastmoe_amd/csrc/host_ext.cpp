@@ -12,6 +12,8 @@
 //       column count, and row-contiguous (is_contiguous()).  table is a bytearray of 16 * E bytes:
 //       the E data addresses (int64; 0 for an expert without rows), then the E row counts.
 //       version_sum is versions(seq) when asked for, else 0.
+//   requires_grad(seq) -> bool
+//       Whether any element is a tensor that requires grad.
 //   versions(seq) -> int
 //       Sum of the tensors' autograd version counters.  Counters never decrease, so the sum
 //       grows whenever any tensor is modified in place.
@@ -142,10 +144,29 @@ PyObject* versions(PyObject*, PyObject* seq) {
   return PyLong_FromLongLong(sum);
 }
 
+PyObject* requires_grad(PyObject*, PyObject* seq) {
+  PyObject* fast = PySequence_Fast(seq, "fastmoe_amd: expected a sequence of tensors");
+  if (!fast) return nullptr;
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(fast);
+  PyObject** items = PySequence_Fast_ITEMS(fast);
+  bool any = false;
+  try {
+    for (Py_ssize_t i = 0; i < n && !any; ++i)
+      any = THPVariable_Check(items[i]) && THPVariable_Unpack(items[i]).requires_grad();
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_ValueError, e.what());
+  }
+  Py_DECREF(fast);
+  if (PyErr_Occurred()) return nullptr;
+  return PyBool_FromLong(any);
+}
+
 PyMethodDef kMethods[] = {
     {"experts", experts, METH_VARARGS,
      "experts(seq, versions=False) -> (hidden, n_rows, max_rows, table, version_sum): validate "
      "the expert buffers and pack their (address, rows) pairs"},
+    {"requires_grad", requires_grad, METH_O,
+     "requires_grad(seq) -> whether any element is a tensor that requires grad"},
     {"versions", versions, METH_O, "versions(seq) -> sum of the tensors' version counters"},
     {nullptr, nullptr, 0, nullptr}};
 

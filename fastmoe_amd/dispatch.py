@@ -31,7 +31,7 @@ import torch
 
 from . import _abi, ops
 from .ops import (_FLOAT_CODES, _INDEX_CODES, _launch_fwd, _on_device, _refuse_autograd_capture,
-                  _require_cuda, _span, _stream_handle, _validate_default,
+                  _require_cuda, _runs_plain, _span, _stream_handle, _validate_default,
                   prepare_metadata_and_plan)
 
 __all__ = ["PermutedTokens", "permute_tokens"]
@@ -90,67 +90,74 @@ def _small_slots() -> int:
     return _SMALL_SLOTS[0]
 
 
+def _permute(x_flat, topk_weights, topk_indices, num_experts, validate):
+    """(permuted rows, sorted gates, counts, reverse map, offsets, slot map) of checked arguments."""
+    lib = _abi.lib()
+    T, D = x_flat.shape
+    k = topk_indices.shape[1]
+    E = int(num_experts)
+    dev = x_flat.device
+    ids = topk_indices.reshape(-1).contiguous()
+    gates = topk_weights.reshape(-1).contiguous()
+    N = T * k
+    counts = torch.empty(E, dtype=torch.int64, device=dev)
+    offsets = torch.empty(E + 1, dtype=torch.int64, device=dev)
+    rev = torch.empty(N, dtype=torch.int64, device=dev)
+    sorted_w = torch.empty(N, dtype=gates.dtype, device=dev)
+    slot_pos = torch.empty(N, dtype=torch.int32, device=dev)
+    status = torch.empty(1, dtype=torch.int32, device=dev)
+    es = x_flat.element_size()
+    out = torch.empty((N, D), dtype=x_flat.dtype, device=dev)
+    x_stride = (x_flat.stride(0) if T > 1 else D) * es
+    whole = N > 0 and D > 0 and ops._TIMER is None  # one call; timed: one per span
+    ws = None
+    if not whole or N > _small_slots():
+        ws = torch.empty(max(lib.fmoe_permute_workspace_bytes(N, E), 256), dtype=torch.uint8,
+                         device=dev)
+    with _on_device(dev):
+        if whole:
+            rc = lib.fmoe_permute(
+                ids.data_ptr(), _INDEX_CODES[ids.dtype], gates.data_ptr(),
+                _FLOAT_CODES[gates.dtype], T, k, E, D * es, x_flat.data_ptr(), x_stride,
+                counts.data_ptr(), offsets.data_ptr(), rev.data_ptr(), sorted_w.data_ptr(),
+                slot_pos.data_ptr(), status.data_ptr(), out.data_ptr(),
+                ws.data_ptr() if ws is not None else None, _stream_handle(dev))
+            _abi.check(rc, "fmoe_permute")
+        else:
+            with _span("permute_build"):
+                rc = lib.fmoe_permute_build(
+                    ids.data_ptr(), _INDEX_CODES[ids.dtype], gates.data_ptr(),
+                    _FLOAT_CODES[gates.dtype], T, k, E, counts.data_ptr(), offsets.data_ptr(),
+                    rev.data_ptr(), sorted_w.data_ptr(), slot_pos.data_ptr(),
+                    status.data_ptr(), ws.data_ptr(), _stream_handle(dev))
+            _abi.check(rc, "fmoe_permute_build")
+            if N and D:
+                with _span("permute_gather"):
+                    rc = lib.fmoe_permute_gather(
+                        slot_pos.data_ptr(), T, k, D * es, x_flat.data_ptr(), x_stride,
+                        out.data_ptr(), _stream_handle(dev))
+                _abi.check(rc, "fmoe_permute_gather")
+    if validate:
+        bad = int(status[0])
+        if bad:
+            raise IndexError(f"fastmoe_amd: {bad} expert ids lie outside [0, {E})")
+    return out, sorted_w, counts, rev, offsets, slot_pos
+
+
 class _TokenPermute(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x_flat, topk_weights, topk_indices, num_experts, validate):
-        lib = _abi.lib()
-        T, D = x_flat.shape
-        k = topk_indices.shape[1]
-        E = int(num_experts)
-        dev = x_flat.device
-        ids = topk_indices.reshape(-1).contiguous()
-        gates = topk_weights.reshape(-1).contiguous()
-        N = T * k
-        counts = torch.empty(E, dtype=torch.int64, device=dev)
-        offsets = torch.empty(E + 1, dtype=torch.int64, device=dev)
-        rev = torch.empty(N, dtype=torch.int64, device=dev)
-        sorted_w = torch.empty(N, dtype=gates.dtype, device=dev)
-        slot_pos = torch.empty(N, dtype=torch.int32, device=dev)
-        status = torch.empty(1, dtype=torch.int32, device=dev)
-        es = x_flat.element_size()
-        out = torch.empty((N, D), dtype=x_flat.dtype, device=dev)
-        x_stride = (x_flat.stride(0) if T > 1 else D) * es
-        whole = N > 0 and D > 0 and ops._TIMER is None  # one call; timed: one per span
-        ws = None
-        if not whole or N > _small_slots():
-            ws = torch.empty(max(lib.fmoe_permute_workspace_bytes(N, E), 256), dtype=torch.uint8,
-                             device=dev)
-        with _on_device(dev):
-            if whole:
-                rc = lib.fmoe_permute(
-                    ids.data_ptr(), _INDEX_CODES[ids.dtype], gates.data_ptr(),
-                    _FLOAT_CODES[gates.dtype], T, k, E, D * es, x_flat.data_ptr(), x_stride,
-                    counts.data_ptr(), offsets.data_ptr(), rev.data_ptr(), sorted_w.data_ptr(),
-                    slot_pos.data_ptr(), status.data_ptr(), out.data_ptr(),
-                    ws.data_ptr() if ws is not None else None, _stream_handle(dev))
-                _abi.check(rc, "fmoe_permute")
-            else:
-                with _span("permute_build"):
-                    rc = lib.fmoe_permute_build(
-                        ids.data_ptr(), _INDEX_CODES[ids.dtype], gates.data_ptr(),
-                        _FLOAT_CODES[gates.dtype], T, k, E, counts.data_ptr(), offsets.data_ptr(),
-                        rev.data_ptr(), sorted_w.data_ptr(), slot_pos.data_ptr(),
-                        status.data_ptr(), ws.data_ptr(), _stream_handle(dev))
-                _abi.check(rc, "fmoe_permute_build")
-                if N and D:
-                    with _span("permute_gather"):
-                        rc = lib.fmoe_permute_gather(
-                            slot_pos.data_ptr(), T, k, D * es, x_flat.data_ptr(), x_stride,
-                            out.data_ptr(), _stream_handle(dev))
-                    _abi.check(rc, "fmoe_permute_gather")
-        if validate:
-            bad = int(status[0])
-            if bad:
-                raise IndexError(f"fastmoe_amd: {bad} expert ids lie outside [0, {E})")
+        outs = _permute(x_flat, topk_weights, topk_indices, num_experts, validate)
+        _, _, counts, rev, offsets, slot_pos = outs
         ctx.save_for_backward(rev, slot_pos)
-        ctx.num_tokens = T
-        ctx.top_k = k
-        ctx.x_dtype, ctx.hidden, ctx.gate_dtype = x_flat.dtype, D, gates.dtype
+        ctx.num_tokens, ctx.top_k = topk_indices.shape
+        ctx.x_dtype, ctx.hidden = x_flat.dtype, x_flat.shape[1]
+        ctx.gate_dtype = topk_weights.dtype
         ctx.mark_non_differentiable(counts, rev, offsets, slot_pos)
         # an output without a gradient arrives as None: autograd would otherwise fill a zero tensor
         # for each of the integer outputs in every backward (four launches)
         ctx.set_materialize_grads(False)
-        return out, sorted_w, counts, rev, offsets, slot_pos
+        return outs
 
     @staticmethod
     def backward(ctx, g_out, g_sorted_w, _g_counts, _g_rev, _g_off, _g_pos):
@@ -229,6 +236,7 @@ def permute_tokens(x_flat: torch.Tensor, topk_indices: torch.Tensor, topk_weight
     if torch.is_grad_enabled():
         _refuse_autograd_capture("the autograd permutation", x_flat,
                                  x_flat.requires_grad or topk_weights.requires_grad)
-    out, sorted_w, counts, rev, offsets, slot_pos = _TokenPermute.apply(
-        x_flat, topk_weights, topk_indices, int(num_experts), _validate_default(validate))
+    args = (x_flat, topk_weights, topk_indices, int(num_experts), _validate_default(validate))
+    run = _permute if _runs_plain((x_flat, topk_weights)) else _TokenPermute.apply
+    out, sorted_w, counts, rev, offsets, slot_pos = run(*args)
     return PermutedTokens(out, counts, rev, sorted_w, offsets, slot_pos)

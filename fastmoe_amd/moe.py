@@ -27,7 +27,8 @@ import torch.nn.functional as F
 
 from .consts import MoEImplementation
 from .dispatch import PermutedTokens, permute_tokens
-from .ops import _apply, _GroupedCombinePermuted, grouped_weighted_scatter_add
+from .ops import (_apply, _combine_forward, _GroupedCombinePermuted, _runs_plain,
+                  grouped_weighted_scatter_add)
 
 __all__ = ["MoEFeedForward", "compute_experts", "gate_and_sort", "unpermute"]
 
@@ -88,8 +89,13 @@ def unpermute(x_out: Union[torch.Tensor, Sequence[torch.Tensor]], reverse_map_in
     if impl == MoEImplementation.FAST:
         if permutation is not None:
             k = permutation.slot_pos.numel() // (B * T) if B * T else 0
-            out = _apply(_GroupedCombinePermuted, (permutation.slot_pos, k), reverse_map_indices,
-                         sorted_weights, (B * T, D), *parts)
+            slots = (permutation.slot_pos, k)
+            if _runs_plain((sorted_weights, *parts)):
+                out = _combine_forward(None, None, None, reverse_map_indices, sorted_weights,
+                                       (B * T, D), parts, False, slots)
+            else:
+                out = _apply(_GroupedCombinePermuted, slots, reverse_map_indices, sorted_weights,
+                             (B * T, D), *parts)
         else:
             out = grouped_weighted_scatter_add(parts, reverse_map_indices, sorted_weights,
                                                (B * T, D))
