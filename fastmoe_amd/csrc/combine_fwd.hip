@@ -411,6 +411,111 @@ __global__ __launch_bounds__(kGroup) void k_fwd_atomic(
     fwd_atomic_body<TX, TO, V, U, true>(src, wf, orow, D, chunk);
 }
 
+// ---- atomic mode with few output rows: a workgroup's rows ordered by token first ----------------
+// k_fwd_atomic sends every product to the memory side, whose atomic rate bounds it.  When the
+// tokens are few, many of a workgroup's rows go to the same one: it takes a share of the rows and
+// a slice of 64 columns, orders its rows by token in LDS (a counting sort; rows out of range are
+// left out), and each of its waves walks a sixteenth of them, summing a token's run in registers
+// and adding it to the output once.  The memory side then sees T + 15 adds per workgroup and
+// column instead of its rows.  A lane holds one column, so that a wave's adds are consecutive (2
+// and 4 columns per lane measured 67 and 198 us where 1 takes 58); 256 workgroups.  The sums start
+// at -0, which a first term replaces exactly; the order of the additions varies, as everywhere in
+// this mode.  us, k_fwd_atomic -> this kernel (one MI355X, three inputs in turn):
+//   T=128, D=1024, N=65536   fp32 216 -> 58, bf16 211 -> 44      T=1000, D=1024, N=65536  212 -> 71
+//   T=16, D=1024, N=65536    221 -> 52                           T=64, D=100, N=131072    83 -> 22
+//   T=300, D=2048, N=131072  815 -> 224                          T=32, D=256, N=4096      9.6 -> 7.4
+// Sums kept in LDS for all T tokens (ds_add_f32) took 341 us at the first of these: a wave's float
+// add to LDS takes about 200 cycles.
+constexpr int kFewThreads = kScanThreads;
+constexpr int kFewWaves = kFewThreads / kWave;
+constexpr int kFewGroups = 256;   // workgroups aimed at
+constexpr int kFewRows = 8192;    // rows per workgroup at most: the sorted list's LDS
+constexpr int kFewTokens = 1024;  // one per thread in the scan
+constexpr int kFewBatch = 16;     // rows in flight per wave
+static_assert(kFewRows <= (1 << 16) && kFewTokens <= (1 << 16), "list entries: token, row");
+
+template <typename TX>
+__global__ __launch_bounds__(kFewThreads) void k_fwd_atomic_few(
+    const int64_t* __restrict__ ptr_table, const int64_t* __restrict__ offsets, int64_t E,
+    const void* __restrict__ idx, int idx_dtype, const void* __restrict__ w, int w_dtype,
+    float* __restrict__ out, int64_t out_stride, uint32_t D, uint32_t N, uint32_t T,
+    uint32_t slices, uint32_t rows_per_group) {
+  using VX = Vec<TX, 1>;
+  __shared__ uint32_t list[kFewRows];  // (token << 16 | row of the share), by token
+  __shared__ int place[kFewTokens];    // rows per token, then the token's next place
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = uniform(tid / kWave);
+  const uint32_t share = blockIdx.x / slices;  // of the rows; its slices are neighbours
+  const uint32_t col = (blockIdx.x - share * slices) * kWave + (uint32_t)lane;
+  const uint32_t beg = share * rows_per_group;  // < N: the host sizes the grid so
+  const uint32_t n = min(rows_per_group, N - beg);
+  place[tid] = 0;
+  __syncthreads();
+  for (uint32_t i = tid; i < n; i += kFewThreads) {
+    const int64_t t = load_index(idx, idx_dtype, beg + i);
+    if (t >= 0 && t < (int64_t)T) atomicAdd(&place[(int)t], 1);
+  }
+  __syncthreads();
+  int rows;
+  const int first = block_exclusive_scan_1024(place[tid], &rows);
+  place[tid] = first;
+  __syncthreads();
+  for (uint32_t i = tid; i < n; i += kFewThreads) {
+    const int64_t t = load_index(idx, idx_dtype, beg + i);
+    if (t >= 0 && t < (int64_t)T) list[atomicAdd(&place[(int)t], 1)] = (uint32_t)t << 16 | i;
+  }
+  __syncthreads();
+
+  const uint32_t row_bytes = D * (uint32_t)sizeof(TX);
+  const uint32_t off = col * (uint32_t)sizeof(TX);  // past the row: zeros from the range check
+  const int per = (rows + kFewWaves - 1) / kFewWaves;
+  const int p1 = min(rows, (wave + 1) * per);
+  float acc = 0.f;
+  int cur = -1;  // the token of acc; none yet
+  auto flush = [&]() {
+    if (cur >= 0 && col < D) unsafeAtomicAdd(out + (int64_t)cur * out_stride + col, acc);
+  };
+  for (int p = wave * per; p < p1; p += kWave) {
+    const int cnt = min(kWave, p1 - p);
+    LaneRecs lr;  // lr.g: the row's token
+    lr.src_lo = lr.src_hi = lr.w_bits = 0;
+    lr.g = -1;
+    if (lane < cnt) {
+      const uint32_t entry = list[p + lane];
+      const int64_t g = beg + (entry & 0xffffu);
+      const int64_t e = expert_of_row(offsets, E, g);
+      const uint64_t src = (uint64_t)ptr_table[e] + (uint64_t)(g - offsets[e]) * row_bytes;
+      lr.src_lo = (uint32_t)src;
+      lr.src_hi = (uint32_t)(src >> 32);
+      lr.w_bits = __float_as_uint(load_weight(w, w_dtype, g));
+      lr.g = (int)(entry >> 16);
+    }
+    for (int i = 0; i < cnt; i += kFewBatch) {
+      typename VX::raw_t a[kFewBatch];
+#pragma unroll
+      for (int r = 0; r < kFewBatch; ++r)
+        a[r] = VX::template ld<FMOE_X_CPOL>(
+            make_rsrc(lr.src(min(i + r, cnt - 1)), i + r < cnt ? row_bytes : 0u), off);
+#pragma unroll
+      for (int r = 0; r < kFewBatch; ++r) {
+        if (i + r < cnt) {  // wave-uniform
+          const int t = lr.row(i + r);
+          if (t != cur) {  // wave-uniform
+            flush();
+            cur = t;
+            acc = -0.f;
+          }
+          float x;
+          VX::cvt(a[r], &x);
+          acc = acc + x * lr.w(i + r);
+        }
+      }
+    }
+  }
+  flush();
+}
+
 // ---- fp32 accumulator of a 16-bit output, and zero-fill of an overwritten output --------------
 // Row-major passes over [T, D]: a thread per 8 consecutive columns of a row, with 16-byte accesses
 // when the rows allow them (VEC: D % 8 == 0 and 16-byte aligned rows), element accesses otherwise.
@@ -746,8 +851,50 @@ static int launch_fwd_v(FwdArgs a) {
   }
 }
 
+// The few-tokens atomic kernel: its geometry, or 0 groups where it does not apply.  It needs at
+// least 4 rows per token in every share, so that the ordering saves atomics, and applies to an
+// fp32 target (a 16-bit output's accumulator among them); a forced tile or grid order of
+// k_fwd_atomic turns it off.
+struct FewGeom {
+  int64_t slices, rows_per_group, groups;
+};
+static FewGeom few_geom(int64_t N, int64_t T, int64_t D) {
+  FewGeom g{};
+  if (T > kFewTokens || N < 4 * T || fmoe_host::opt(fmoe_host::kOptFwdAtomicTile) != 0 ||
+      fmoe_host::opt(fmoe_host::kOptAtomicOrder) != 0)
+    return g;
+  g.slices = (D + kWave - 1) / kWave;
+  int64_t shares = std::max<int64_t>(1, kFewGroups / g.slices);
+  shares = std::min<int64_t>(shares, N / (4 * T));
+  shares = std::max<int64_t>(shares, (N + kFewRows - 1) / kFewRows);
+  g.rows_per_group = (N + shares - 1) / shares;
+  shares = (N + g.rows_per_group - 1) / g.rows_per_group;  // none of them empty
+  g.groups = shares * g.slices;
+  return g;
+}
+
+template <typename TX>
+static int launch_few(const FwdArgs& a, const FewGeom& g) {
+  if (g.groups >= (int64_t(1) << 31)) {
+    fmoe_host::set_error("fmoe_combine_fwd(atomic): grid too large (%lld workgroups)",
+                         (long long)g.groups);
+    return FMOE_ERANGE;
+  }
+  hipLaunchKernelGGL((k_fwd_atomic_few<TX>), dim3((unsigned)g.groups), dim3(kFewThreads), 0, a.s,
+                     a.ptr_table, a.offsets, a.E, a.idx, a.idx_dtype, a.w, a.w_dtype,
+                     static_cast<float*>(a.out), a.out_stride, (uint32_t)a.D, (uint32_t)a.N,
+                     (uint32_t)a.T, (uint32_t)g.slices, (uint32_t)g.rows_per_group);
+  return fmoe_host::check_launch("fmoe_combine_fwd(atomic, few tokens)");
+}
+
 template <typename TX, typename TO>
 static int launch_fwd_t(const FwdArgs& a) {
+  if constexpr (sizeof(TO) == 4) {
+    if (a.mode != FMOE_MODE_DET) {
+      const FewGeom g = few_geom(a.N, a.T, a.D);
+      if (g.groups > 0) return launch_few<TX>(a, g);
+    }
+  }
   constexpr int V = vec16<TX>();
   const int ob = (int)sizeof(TO) == 4 ? 4 : 2;
   const int64_t vb = (int64_t)V * ob;  // bytes of one output vector

@@ -1,0 +1,58 @@
+"""The atomic forward's few-tokens kernel (rows ordered by token within a workgroup): within the
+bound of a reordered fp32 sum of the C oracle's result, at the edges of its rule and shares."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import fastmoe_amd
+from tests.helpers import abs_sum, oracle_fwd, reorder_tol, to_np, within_one_ulp16
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("T,counts,D,dtype,opts", [
+    (1, [1, 3], 1, torch.float32, {}),
+    (1, [9000], 65, torch.float32, {}),                          # one token, two shares
+    (16, [30, 0, 33], 64, torch.bfloat16, {"bad": True}),        # 63 rows: below 4 per token
+    (16, [31, 0, 33], 64, torch.bfloat16, {"bad": True}),        # 64: the rule's edge
+    (128, [5000, 3192, 1], 100, torch.float32, {"int32": True}),  # shares that end inside an expert
+    (1024, [4096], 200, torch.float32, {}),                      # the most tokens
+    (1025, [4100], 200, torch.float32, {}),                      # one more: k_fwd_atomic
+    (7, [16385], 130, torch.float16, {"w16": True}),             # 3 shares of at most 8192 rows
+    (3, [40, 80], 16400, torch.bfloat16, {}),                    # more slices than workgroups aimed at
+])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_few_tokens_match_the_oracle(T, counts, D, dtype, opts, accumulate):
+    gen = torch.Generator().manual_seed(T + D)
+    experts = [torch.randn(n, D, generator=gen).to(dtype) for n in counts]
+    N = sum(counts)
+    idx = torch.randint(0, T, (N,), generator=gen)
+    if opts.get("bad"):
+        idx[::5] = T + 1
+        idx[1::9] = -2
+    w = torch.rand(N, generator=gen)
+    if opts.get("w16"):
+        w = w.to(dtype)
+    wd, xd = w.to(DEV), [x.to(DEV) for x in experts]
+    idxd = (idx.int() if opts.get("int32") else idx).to(DEV)
+    init = torch.randn(T, D, generator=gen).to(dtype) if accumulate else None
+    if accumulate:
+        got = init.to(DEV)
+        fastmoe_amd.grouped_weighted_scatter_add(xd, idxd, wd, (T, D), out=got, mode="atomic")
+        acc0 = init.float().numpy()
+    else:
+        got = fastmoe_amd.grouped_weighted_scatter_add(xd, idxd, wd, (T, D), mode="atomic")
+        acc0 = None
+    want, acc, _ = oracle_fwd(experts, idx, w, T, dtype, acc_init=acc0)
+    scale = abs_sum(experts, idx, w, T) + (np.abs(init.float().numpy()) if accumulate else 0.0)
+    valid = idx[(idx >= 0) & (idx < T)]
+    n = int(torch.bincount(valid, minlength=T).max()) + 1
+    if dtype == torch.float32:
+        assert np.all(np.abs(to_np(got).astype(np.float64) - acc) <= reorder_tol(n, scale))
+    else:
+        g = got.float().cpu().numpy()
+        wantf = torch.from_numpy(want.view(np.int16)).view(dtype).float().numpy()
+        assert np.all(within_one_ulp16(g, wantf, dtype, n, scale))
