@@ -209,10 +209,17 @@ __global__ __launch_bounds__(kGroup) void k_slots_bwd(const int32_t* __restrict_
 // For at most kSmallRows rows the plan is not worth its own launch.  Every workgroup stages the
 // token id of each row in LDS (-1 for an index outside [0, T)); a wave owns one (token, column
 // chunk) unit as in k_fwd_det and finds the token's rows by ballots over the staged ids in
-// ascending row order, compacting them through a 128-entry window and taking them 64 at a time.
+// ascending row order, 256 ids per step (four per lane in one 16-byte LDS read), compacting them
+// through a window and taking them 64 at a time.  With 64 ids per step the scan bound the kernel
+// from about 1024 rows; the kernel in us (bf16, T, D, top-k; launches in a graph), plan + k_fwd_det
+// beside it:  64, 7168, 8: 6.0 (11.5)   128, 7168, 8: 7.1 (14.2)   256, 7168, 8: 9.7 (14.6)
+// 512, 7168, 8: 17.2 (18.1)   1024, 1024, 4: 10.0 (11.2)   4096, 2048, 1: 15.5 (13.8).
 // Lanes look up their row's expert in an LDS copy of the argument table.  The rows are added in
 // ascending g with k_fwd_det's arithmetic, so the result is the same, bit for bit.
 static_assert(kMetaChunk == kGroup, "one expert per thread copies the argument table");
+constexpr int kSmallIds = 4;                   // staged ids per lane per step: one 16-byte LDS read
+constexpr int kSmallStep = kWave * kSmallIds;  // ids per step
+static_assert(kSmallRows % kSmallStep == 0, "whole steps");
 template <typename TX, typename TO, int V, int U, bool AL>
 __global__ __launch_bounds__(kGroup) void k_fwd_small(const HostTable meta,
                                                       const void* __restrict__ idx, int idx_dtype,
@@ -224,8 +231,8 @@ __global__ __launch_bounds__(kGroup) void k_fwd_small(const HostTable meta,
   using VO = Vec<TO, V>;
   constexpr int CW = kWave * V * U;
   constexpr int R = AL ? 4 : 1;  // rows per batch of loads (one at a time for element loads)
-  __shared__ int tok[kSmallRows];
-  __shared__ int win[kWavesPerGroup][2 * kWave];
+  __shared__ __attribute__((aligned(16))) uint32_t tok[kSmallRows];
+  __shared__ int win[kWavesPerGroup][kWave + kSmallStep];
   __shared__ int off_lds[kMetaChunk + 1];
   __shared__ uint64_t ptr_lds[kMetaChunk];
   __shared__ int invalid;
@@ -236,11 +243,12 @@ __global__ __launch_bounds__(kGroup) void k_fwd_small(const HostTable meta,
   small_table_to_lds(meta, off_lds, ptr_lds);
   __syncthreads();
   int bad = 0;
-  for (uint32_t g = tid; g < N; g += kGroup) {
-    const int64_t v = load_index(idx, idx_dtype, g);
+  const uint32_t padded = (N + kSmallStep - 1) / kSmallStep * kSmallStep;
+  for (uint32_t g = tid; g < padded; g += kGroup) {
+    const int64_t v = g < N ? load_index(idx, idx_dtype, g) : -1;
     const bool ok = v >= 0 && v < (int64_t)T;
-    tok[g] = ok ? (int)v : -1;
-    bad += ok ? 0 : 1;
+    tok[g] = ok ? (uint32_t)v : 0xffffffffu;
+    bad += ok || g >= N ? 0 : 1;
   }
   if (blockIdx.x == 0 && bad) atomicAdd(&invalid, bad);
   __syncthreads();
@@ -273,17 +281,32 @@ __global__ __launch_bounds__(kGroup) void k_fwd_small(const HostTable meta,
     }
     int have = 0;  // rows in the window (wave-uniform)
     int seen = 0;
-    for (uint32_t base = 0; base < N; base += kWave) {
-      const uint32_t g = base + (uint32_t)lane;
-      const bool hit = g < N && tok[g] == (int)t;
-      const uint64_t m = __ballot(hit);
-      if (hit) win[wave][have + lanes_below(m)] = (int)g;
-      have += __builtin_popcountll(m);
-      const bool last = base + kWave >= N;
-      while (have >= kWave || (last && have > 0)) {
-        const int cnt = have < kWave ? have : kWave;
+    for (uint32_t base = 0; base < padded; base += kSmallStep) {
+      // a lane's kSmallIds consecutive ids, then the next lane's: ascending rows
+      const u32x4 id = *reinterpret_cast<const u32x4*>(&tok[base + (uint32_t)lane * kSmallIds]);
+      uint64_t m[kSmallIds];
+      uint64_t any = 0;
+#pragma unroll
+      for (int r = 0; r < kSmallIds; ++r) {
+        m[r] = __ballot(id[r] == t);
+        any |= m[r];
+      }
+      const bool last = base + kSmallStep >= padded;
+      if (any) {  // wave-uniform
+        int at = have;
+#pragma unroll
+        for (int r = 0; r < kSmallIds; ++r) at += lanes_below(m[r]);
+#pragma unroll
+        for (int r = 0; r < kSmallIds; ++r) {
+          if (id[r] == t) win[wave][at++] = (int)(base + (uint32_t)lane * kSmallIds + r);
+          have += __builtin_popcountll(m[r]);
+        }
+      }
+      int head = 0;
+      while (have - head >= kWave || (last && have > head)) {
+        const int cnt = min(have - head, kWave);
         LaneRecs lr;
-        lr.g = lane < cnt ? win[wave][lane] : 0;
+        lr.g = lane < cnt ? win[wave][head + lane] : 0;
         if (lane < cnt) {
           const int e = expert_of_row32(off_lds, ne, lr.g);
           const uint64_t src =
@@ -294,12 +317,15 @@ __global__ __launch_bounds__(kGroup) void k_fwd_small(const HostTable meta,
         } else {
           lr.src_lo = lr.src_hi = lr.w_bits = 0;
         }
-        const int rest = have - cnt;  // at most 63 rows carried to the window's front
-        const int carry = lane < rest ? win[wave][cnt + lane] : 0;
-        if (lane < rest) win[wave][lane] = carry;
-        have = rest;
+        head += cnt;
         seen += cnt;
         add_rows<TX, V, U, R, AL>(lr, cnt, xrow_bytes, xoff, acc);
+      }
+      if (head > 0) {  // at most 63 rows carried to the window's front
+        const int rest = have - head;
+        const int carry = lane < rest ? win[wave][head + lane] : 0;
+        if (lane < rest) win[wave][lane] = carry;
+        have = rest;
       }
     }
     if (accumulate && seen == 0) continue;  // nothing routed here: out keeps its contents

@@ -563,18 +563,27 @@ def _launch_fwd(meta: GroupedMetadata, mode: int, plan: Optional[torch.Tensor],
 
 # The one-launch small path (fmoe_combine_fwd_small / fmoe_combine_bwd_small): deterministic calls
 # of at most fmoe_combine_small_max_rows() rows over at most 256 experts, with no plan.  A training
-# step is two launches instead of four (metadata + plan, forward, grad_X pass, grad_w pass), and a
+# step is two launches instead of four (metadata + plan, forward, grad_w pass, grad_X pass), and a
 # forward saves the plan's dependent launch.  Each forward wave scans the token id of every row, so
-# the cost grows with T * N: it is taken while T * N <= _SMALL_SCAN_LIMIT (graph-replayed steps on
-# one MI355X, planned -> small: fwd+bwd 17.6 -> 15.3 us at T=256, D=512, top-2, fp32 and 24.3 ->
-# 18.9 us at T=64, D=7168, top-8, bf16; forward 19.0 -> 14.8 us at T=128, D=16384, top-8; past
-# the limit, fwd+bwd 31.9 -> 33.7 us at T=256, D=7168, top-8).
+# the cost grows with T * N: calls with T * N <= _SMALL_ALWAYS take it, and up to _SMALL_SCAN_LIMIT
+# those of at most _SMALL_TOKENS tokens (the waves of its grid).  Its backward writes grad_X between
+# its reads, which the planned passes keep apart, so a call that records a backward takes it beyond
+# _SMALL_ALWAYS only while its rows are at most _SMALL_STEP_BYTES.  Launches in graphs on one MI355X, bf16, forward + backward in us, planned -> small:
+#   T=64, D=7168, top-8     11.5 + 9.6 ->  6.0 + 7.8     T=1024, D=1024, top-4   11.2 + 7.0 -> 10.0 + 6.0
+#   T=256, D=7168, top-8   14.6 + 12.4 ->  9.7 + 14.6    T=256, D=16384, top-8  19.0 + 24.4 -> 15.7 + 31.6
+#   T=512, D=4096, top-6   13.6 + 11.7 -> 10.1 + 12.6    T=512, D=7168, top-8   18.1 + 22.6 -> 17.2 + 27.2
+# and past the scan's limit T=4096, D=2048, top-1: 13.8 -> 15.5 forward.
 _SMALL_MAX_EXPERTS = 256
-_SMALL_SCAN_LIMIT = 1 << 17
+_SMALL_ALWAYS = 1 << 17
+_SMALL_SCAN_LIMIT = 1 << 22
+_SMALL_TOKENS = 4096
+_SMALL_STEP_BYTES = 32 << 20
 _SMALL_MAX_ROWS: list = []
 
 
-def _use_small(rows: int, num_tokens: int, num_experts: int) -> bool:
+def _use_small(rows: int, num_tokens: int, num_experts: int, step_bytes: int = 0) -> bool:
+    """Whether a deterministic call takes the small path; ``step_bytes``: the bytes of its expert
+    rows if it records a backward, else 0."""
     choice = _abi.option("small")
     if choice == 1 or _abi.option("plan") != 0 or num_experts > _SMALL_MAX_EXPERTS or rows < 1:
         return False
@@ -582,7 +591,10 @@ def _use_small(rows: int, num_tokens: int, num_experts: int) -> bool:
         _SMALL_MAX_ROWS.append(int(_abi.lib().fmoe_combine_small_max_rows()))
     if rows > _SMALL_MAX_ROWS[0]:
         return False
-    return choice == 2 or rows * num_tokens <= _SMALL_SCAN_LIMIT
+    scan = rows * num_tokens
+    return (choice == 2 or scan <= _SMALL_ALWAYS
+            or (scan <= _SMALL_SCAN_LIMIT and num_tokens <= _SMALL_TOKENS
+                and step_bytes <= _SMALL_STEP_BYTES))
 
 
 def _launch_fwd_small(tables, num_experts: int, idx: torch.Tensor, w: torch.Tensor,
@@ -669,7 +681,8 @@ def _combine_forward(ctx, mode: Optional[str], validate: Optional[bool], indices
         meta = _RawMeta(ex)
         _run_metadata(ex, meta)
         out = torch.zeros(shape, dtype=dtype, device=dev)
-    elif code == _abi.MODE_DET and _use_small(rows, T, ex.num):
+    elif code == _abi.MODE_DET and _use_small(
+            rows, T, ex.num, rows * hidden * _ELEM_BYTES[dtype] if ctx is not None else 0):
         # one launch, no plan; the backward is one launch too
         small = ex.host_tables()
         out = torch.empty(shape, dtype=dtype, device=dev)
