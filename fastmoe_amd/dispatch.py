@@ -233,10 +233,9 @@ def permute_tokens(x_flat: torch.Tensor, topk_indices: torch.Tensor, topk_weight
         raise ValueError(f"fastmoe_amd: num_experts must be in [1, 4096], got {num_experts}")
     if len({x_flat.device, topk_indices.device, topk_weights.device}) != 1:
         raise ValueError("fastmoe_amd: x_flat, topk_indices and topk_weights must share a device")
-    if torch.is_grad_enabled():
-        _refuse_autograd_capture("the autograd permutation", x_flat,
-                                 x_flat.requires_grad or topk_weights.requires_grad)
+    records = torch.is_grad_enabled() and (x_flat.requires_grad or topk_weights.requires_grad)
+    _refuse_autograd_capture("the autograd permutation", x_flat, records)
     args = (x_flat, topk_weights, topk_indices, int(num_experts), _validate_default(validate))
-    run = _permute if _runs_plain((x_flat, topk_weights)) else _TokenPermute.apply
+    run = _permute if not records and _runs_plain((x_flat, topk_weights)) else _TokenPermute.apply
     out, sorted_w, counts, rev, offsets, slot_pos = run(*args)
     return PermutedTokens(out, counts, rev, sorted_w, offsets, slot_pos)

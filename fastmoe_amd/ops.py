@@ -927,10 +927,11 @@ def grouped_weighted_scatter_add(expert_tensors, indices, weights, out_shape, ou
     if out is not None:
         return _launch_grouped_kernel(expert_tensors, indices, weights, out, metadata=metadata,
                                       mode=mode, validate=validate)
-    expert_tensors = tuple(expert_tensors)
-    if _runs_plain((weights, *expert_tensors)):
-        return _combine_forward(None, mode, validate, indices, weights, out_shape, expert_tensors,
-                                False)
+    if not (torch.is_grad_enabled() and weights.requires_grad):  # else it records: no need to look
+        expert_tensors = tuple(expert_tensors)
+        if _runs_plain((weights, *expert_tensors)):
+            return _combine_forward(None, mode, validate, indices, weights, out_shape,
+                                    expert_tensors, False)
     if mode is None and validate is None:
         return _apply(GroupedWeightedScatterAdd, indices, weights, out_shape, *expert_tensors)
     return _apply(_GroupedCombineWithOptions, (mode, validate), indices, weights, out_shape,
