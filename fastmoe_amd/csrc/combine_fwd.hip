@@ -740,6 +740,7 @@ struct FwdArgs {
 //   4096, 16384, 8 (128 MiB)    217.2 / 212.2     635.9 / 613.4
 //   16384, 4096, 6 (128 MiB)    167.1 / 160.0     483.8 / 463.8
 //   6144, 16384, 8 (192 MiB)    324.4 / 319.7     930.4 / 922.9
+//   32768, 16384, 2 (1 GiB)     520.5 / 523.2    1677.7 / 1623.8
 // The line lies where the forward alone gains too; below it a program that only runs forwards
 // keeps the shorter one.  An accumulating call has just read its output and the caller has just
 // written it, so its lines are in the cache: fp32, 256 MiB, zero-fill + call 291.6 us temporal,
