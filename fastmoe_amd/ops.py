@@ -814,11 +814,11 @@ def _runs_plain(tensors) -> bool:
     nothing else watches the call -- no functorch transform, no forward-mode level (whose tangents
     a Function without a jvp refuses), no tracing and no compiler.  ``apply`` costs about 0.2 us per
     expert tensor: 64 us of the 69 us that a decoding call with 256 experts takes."""
-    return ((not torch.is_grad_enabled() or not _host().requires_grad(tensors))
+    return (not torch.compiler.is_compiling()  # first: the compiler does not trace the others
             and not torch._C._are_functorch_transforms_active()
             and forward_ad._current_level < 0
             and torch._C._get_tracing_state() is None
-            and not torch.compiler.is_compiling())
+            and (not torch.is_grad_enabled() or not _host().requires_grad(tensors)))
 
 
 def _apply(fn, *args):
