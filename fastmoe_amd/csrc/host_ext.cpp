@@ -14,6 +14,9 @@
 //       version_sum is versions(seq) when asked for, else 0.
 //   requires_grad(seq) -> bool
 //       Whether any element is a tensor that requires grad.
+//   wrapped(seq) -> bool
+//       Whether any element is a tensor without storage of its own: a wrapper, as a functorch
+//       transform makes them (and leaves them to a caller that keeps one).
 //   versions(seq) -> int
 //       Sum of the tensors' autograd version counters.  Counters never decrease, so the sum
 //       grows whenever any tensor is modified in place.
@@ -144,7 +147,9 @@ PyObject* versions(PyObject*, PyObject* seq) {
   return PyLong_FromLongLong(sum);
 }
 
-PyObject* requires_grad(PyObject*, PyObject* seq) {
+// Whether `pred` holds for any tensor among the elements.
+template <typename Pred>
+PyObject* any_tensor(PyObject* seq, Pred pred) {
   PyObject* fast = PySequence_Fast(seq, "fastmoe_amd: expected a sequence of tensors");
   if (!fast) return nullptr;
   const Py_ssize_t n = PySequence_Fast_GET_SIZE(fast);
@@ -152,7 +157,7 @@ PyObject* requires_grad(PyObject*, PyObject* seq) {
   bool any = false;
   try {
     for (Py_ssize_t i = 0; i < n && !any; ++i)
-      any = THPVariable_Check(items[i]) && THPVariable_Unpack(items[i]).requires_grad();
+      any = THPVariable_Check(items[i]) && pred(THPVariable_Unpack(items[i]));
   } catch (const std::exception& e) {
     PyErr_SetString(PyExc_ValueError, e.what());
   }
@@ -161,12 +166,22 @@ PyObject* requires_grad(PyObject*, PyObject* seq) {
   return PyBool_FromLong(any);
 }
 
+PyObject* requires_grad(PyObject*, PyObject* seq) {
+  return any_tensor(seq, [](const at::Tensor& t) { return t.requires_grad(); });
+}
+
+PyObject* wrapped(PyObject*, PyObject* seq) {
+  return any_tensor(seq, [](const at::Tensor& t) { return !t.has_storage(); });
+}
+
 PyMethodDef kMethods[] = {
     {"experts", experts, METH_VARARGS,
      "experts(seq, versions=False) -> (hidden, n_rows, max_rows, table, version_sum): validate "
      "the expert buffers and pack their (address, rows) pairs"},
     {"requires_grad", requires_grad, METH_O,
      "requires_grad(seq) -> whether any element is a tensor that requires grad"},
+    {"wrapped", wrapped, METH_O,
+     "wrapped(seq) -> whether any element is a tensor without storage of its own"},
     {"versions", versions, METH_O, "versions(seq) -> sum of the tensors' version counters"},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -236,6 +236,7 @@ def permute_tokens(x_flat: torch.Tensor, topk_indices: torch.Tensor, topk_weight
     records = torch.is_grad_enabled() and (x_flat.requires_grad or topk_weights.requires_grad)
     _refuse_autograd_capture("the autograd permutation", x_flat, records)
     args = (x_flat, topk_weights, topk_indices, int(num_experts), _validate_default(validate))
-    run = _permute if not records and _runs_plain((x_flat, topk_weights)) else _TokenPermute.apply
-    out, sorted_w, counts, rev, offsets, slot_pos = run(*args)
+    plain = not records and _runs_plain((x_flat, topk_weights, topk_indices))
+    outs = _permute(*args) if plain else _TokenPermute.apply(*args)
+    out, sorted_w, counts, rev, offsets, slot_pos = outs
     return PermutedTokens(out, counts, rev, sorted_w, offsets, slot_pos)

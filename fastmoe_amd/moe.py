@@ -90,7 +90,7 @@ def unpermute(x_out: Union[torch.Tensor, Sequence[torch.Tensor]], reverse_map_in
         if permutation is not None:
             k = permutation.slot_pos.numel() // (B * T) if B * T else 0
             slots = (permutation.slot_pos, k)
-            if _runs_plain((sorted_weights, *parts)):
+            if _runs_plain((reverse_map_indices, sorted_weights, *parts)):
                 out = _combine_forward(None, None, None, reverse_map_indices, sorted_weights,
                                        (B * T, D), parts, False, slots)
             else:

@@ -809,15 +809,18 @@ def _combine_backward(ctx, grad_output, needs_w: bool, needs_x: Sequence[bool]):
 
 
 def _runs_plain(tensors) -> bool:
-    """Whether a call on ``tensors`` may run its forward directly instead of through
-    ``Function.apply``: nothing would be recorded (grad mode off, or no tensor requires grad) and
-    nothing else watches the call -- no functorch transform, no forward-mode level (whose tangents
-    a Function without a jvp refuses), no tracing and no compiler.  ``apply`` costs about 0.2 us per
-    expert tensor: 64 us of the 69 us that a decoding call with 256 experts takes."""
+    """Whether a call may run its forward directly instead of through ``Function.apply``, given
+    every tensor that ``apply`` would take: nothing would be recorded (grad mode off, or no tensor
+    requires grad) and nothing else watches the call -- no functorch transform, no forward-mode
+    level (whose tangents a Function without a jvp refuses), no tracing and no compiler -- and no
+    argument is a wrapper that escaped from a finished transform, which ``apply`` unwraps.  ``apply``
+    costs about 0.2 us per expert tensor: 64 us of the 69 us that a decoding call with 256 experts
+    takes."""
     return (not torch.compiler.is_compiling()  # first: the compiler does not trace the others
             and not torch._C._are_functorch_transforms_active()
             and forward_ad._current_level < 0
             and torch._C._get_tracing_state() is None
+            and not _host().wrapped(tensors)
             and (not torch.is_grad_enabled() or not _host().requires_grad(tensors)))
 
 
@@ -929,7 +932,7 @@ def grouped_weighted_scatter_add(expert_tensors, indices, weights, out_shape, ou
                                       mode=mode, validate=validate)
     if not (torch.is_grad_enabled() and weights.requires_grad):  # else it records: no need to look
         expert_tensors = tuple(expert_tensors)
-        if _runs_plain((weights, *expert_tensors)):
+        if _runs_plain((indices, weights, *expert_tensors)):
             return _combine_forward(None, mode, validate, indices, weights, out_shape,
                                     expert_tensors, False)
     if mode is None and validate is None:
