@@ -295,6 +295,9 @@ __global__ __launch_bounds__(kPermBlockLarge) void k_perm_place(
   __syncthreads();
   if (live) {
     const int pos = first[key] + in_block;
+    // The ranks are of the ids that k_perm_rank read: ids overwritten since (by another stream, or
+    // a caller whose buffers overlap) give places past the end, which are never written.
+    if (pos < 0 || pos >= N) return;
     rev[pos] = i / k;
     sorted_gates[pos] = gates[i];
     slot_pos[i] = pos;

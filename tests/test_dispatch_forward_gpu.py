@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import fastmoe_amd
+from fastmoe_amd import _abi
 from oracle import cref
 from tests.helpers import to_np
 
@@ -58,3 +59,37 @@ def test_permutation_matches_the_oracle(T, k, E, D, dtype, opts):
     if opts.get("bad"):
         with pytest.raises(IndexError):
             fastmoe_amd.permute_tokens(xd, ids.to(DEV), gates.to(DEV), E, validate=True)
+
+
+@pytest.mark.parametrize("E,block", [(1024, 1024), (1025, 256)])  # rank + place; rank + scan + fill
+def test_ids_overwritten_after_ranking_write_nothing_outside(E, block):
+    """The ids lie where the ranking kernel stores its ranks, so the kernel that places the slots
+    reads the ranks as ids.  All ids are 0: slot i's rank r = i mod block is its new id, and for
+    r > 0 expert r begins at row N, past the outputs.  Only r == 0 has a place; nothing else is
+    written."""
+    T, k = 1024, 3
+    N, guard = T * k, 2048
+    nb = N // block
+    rank_at = (nb * (E + 1) * 4 + 255) // 256 * 256  # block counts first, then the ranks
+    lib = _abi.lib()
+    nbytes = lib.fmoe_permute_workspace_bytes(N, E)
+    assert rank_at + N * 4 <= nbytes
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device=DEV)  # ids: all 0
+    gates = torch.rand(N, device=DEV)
+    counts = torch.empty(E, dtype=torch.int64, device=DEV)
+    offsets = torch.empty(E + 1, dtype=torch.int64, device=DEV)
+    status = torch.empty(1, dtype=torch.int32, device=DEV)
+    rev = torch.full((N + guard,), -7, dtype=torch.int64, device=DEV)
+    sorted_gates = torch.full((N + guard,), -7.0, device=DEV)
+    slot_pos = torch.full((N + guard,), -7, dtype=torch.int32, device=DEV)
+    rc = lib.fmoe_permute_build(
+        ws.data_ptr() + rank_at, _abi.I32, gates.data_ptr(), _abi.F32, T, k, E, counts.data_ptr(),
+        offsets.data_ptr(), rev.data_ptr(), sorted_gates.data_ptr(), slot_pos.data_ptr(),
+        status.data_ptr(), ws.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    _abi.check(rc, "fmoe_permute_build")
+    at = torch.arange(0, N, block, device=DEV)
+    for got, want in ((rev, at // k), (sorted_gates, gates[at]), (slot_pos, at.int())):
+        expect = torch.full_like(got, -7)
+        expect[at] = want.to(got.dtype)
+        assert torch.equal(got, expect)
+    assert int(counts[0]) == N and int(status) == 0
