@@ -459,6 +459,7 @@ constexpr int kFewRows = 8192;    // rows per workgroup at most: the sorted list
 constexpr int kFewTokens = 1024;  // one per thread in the scan
 constexpr int kFewBatch = 16;     // rows in flight per wave
 static_assert(kFewRows <= (1 << 16) && kFewTokens <= (1 << 16), "list entries: token, row");
+static_assert(kFewRows % kFewThreads == 0, "a thread keeps the tokens of its rows in registers");
 
 template <typename TX>
 __global__ __launch_bounds__(kFewThreads) void k_fwd_atomic_few(
@@ -478,19 +479,30 @@ __global__ __launch_bounds__(kFewThreads) void k_fwd_atomic_few(
   const uint32_t n = min(rows_per_group, N - beg);
   place[tid] = 0;
   __syncthreads();
-  for (uint32_t i = tid; i < n; i += kFewThreads) {
-    const int64_t t = load_index(idx, idx_dtype, beg + i);
-    if (t >= 0 && t < (int64_t)T) atomicAdd(&place[(int)t], 1);
+  // A row's index is read once and counted and placed from a register: the list has a place for
+  // every row that was counted, whatever another stream does to the indices meanwhile.
+  int tok[kFewRows / kFewThreads];  // -1: out of range, or no such row
+#pragma unroll
+  for (int j = 0; j < kFewRows / kFewThreads; ++j) {
+    const uint32_t i = (uint32_t)(tid + j * kFewThreads);
+    tok[j] = -1;
+    if (i < n) {
+      const int64_t t = load_index(idx, idx_dtype, beg + i);
+      if (t >= 0 && t < (int64_t)T) tok[j] = (int)t;
+    }
   }
+#pragma unroll
+  for (int j = 0; j < kFewRows / kFewThreads; ++j)
+    if (tok[j] >= 0) atomicAdd(&place[tok[j]], 1);
   __syncthreads();
   int rows;
   const int first = block_exclusive_scan_1024(place[tid], &rows);
   place[tid] = first;
   __syncthreads();
-  for (uint32_t i = tid; i < n; i += kFewThreads) {
-    const int64_t t = load_index(idx, idx_dtype, beg + i);
-    if (t >= 0 && t < (int64_t)T) list[atomicAdd(&place[(int)t], 1)] = (uint32_t)t << 16 | i;
-  }
+#pragma unroll
+  for (int j = 0; j < kFewRows / kFewThreads; ++j)
+    if (tok[j] >= 0)
+      list[atomicAdd(&place[tok[j]], 1)] = (uint32_t)tok[j] << 16 | (uint32_t)(tid + j * kFewThreads);
   __syncthreads();
 
   const uint32_t row_bytes = D * (uint32_t)sizeof(TX);

@@ -56,3 +56,25 @@ def test_few_tokens_match_the_oracle(T, counts, D, dtype, opts, accumulate):
         g = got.float().cpu().numpy()
         wantf = torch.from_numpy(want.view(np.int16)).view(dtype).float().numpy()
         assert np.all(within_one_ulp16(g, wantf, dtype, n, scale))
+
+
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_indices_that_change_during_the_call_lose_no_row(dtype):
+    """Another stream keeps swapping the indices between two valid routings: which of the two a row
+    takes is open, but each row is added exactly once (rows of ones, unit gates: every column sums
+    to N, which fp32 holds exactly)."""
+    T, N, D = 128, 65536, 64
+    routes = [torch.full((N,), t, dtype=dtype, device=DEV) for t in (0, T - 1)]
+    idx = routes[0].clone()
+    x, w = torch.ones(N, D, device=DEV), torch.ones(N, device=DEV)
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream())
+    outs = []
+    for i in range(20):
+        with torch.cuda.stream(other):
+            for j in range(8):
+                idx.copy_(routes[(i + j) % 2])
+        outs.append(fastmoe_amd.weighted_scatter_add(x, idx, w, (T, D), mode="atomic"))
+    torch.cuda.synchronize()
+    for out in outs:
+        assert bool((out.sum(0) == N).all()) and not bool(out[1:T - 1].any())
