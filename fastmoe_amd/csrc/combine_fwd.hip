@@ -890,16 +890,31 @@ static int launch_fwd_v(FwdArgs a) {
   }
 }
 
-// The few-tokens atomic kernel: its geometry, or 0 groups where it does not apply.  It needs at
-// least 4 rows per token in every share, so that the ordering saves atomics, and applies to an
-// fp32 target (a 16-bit output's accumulator among them); a forced tile or grid order of
+// The few-tokens atomic kernel: its geometry, or 0 groups where it is not taken.  It takes an fp32
+// target (a 16-bit output's accumulator among them) of at most kFewTokens rows.  Its shares hold 4
+// rows per token or more, so that the ordering saves atomics; where that leaves few workgroups, or
+// little work, the ordering costs more than the atomics of k_fwd_atomic, which spreads the same rows
+// over the whole device.  So the rule asks for 64 workgroups and for N * D >= 2^22, 2^20 from 96
+// workgroups, or 2^19 from 256 rows per token, whose atomics queue at an address.  us, k_fwd_atomic /
+// this kernel, fp32, whole calls (one MI355X, three inputs in turn):
+//   workgroups: T=1024, N=6144, D=64: 1, 7.9 / 65     T=1024, N=8192, D=512: 16, 21.0 / 51.9
+//     T=1024, N=16384, D=512: 32, 34.7 / 53.5         T=512, N=6144, D=1024: 48, 28.3 / 31.3
+//     T=512, N=8192, D=1024: 64, 35.0 / 31.9          T=256, N=1536, D=4096: 64, 28.9 / 26.0
+//     T=512, N=6144, D=2048: 96, 48.5 / 34.1          T=1024, N=16384, D=2048: 128, 113 / 60.1
+//   work, 64 workgroups: 2^20 (T=64, N=1024, D=1024) 10.0 / 11.2; 2^21 (T=128, N=1024, D=2048)
+//     13.5 / 13.7; 2^22 (T=256, N=2048, D=2048) 21.6 / 20.4
+//   work, 128 and more: 2^19 (T=16, N=256, D=2048) 9.6 / 10.2; 2^20 (T=16, N=512, D=2048) 12.1 / 10.5
+//   256 rows per token: T=1, N=256, D=1024 14.1 / 15.1, D=2048 16.7 / 12.2
+// Option "fwd_atomic_few": 1 = never, 2 = whenever the tokens fit.  A forced tile or grid order of
 // k_fwd_atomic turns it off.
 struct FewGeom {
   int64_t slices, rows_per_group, groups;
 };
 static FewGeom few_geom(int64_t N, int64_t T, int64_t D) {
   FewGeom g{};
-  if (T > kFewTokens || N < 4 * T || fmoe_host::opt(fmoe_host::kOptFwdAtomicTile) != 0 ||
+  const int64_t choice = fmoe_host::opt(fmoe_host::kOptAtomicFew);
+  if (N < 1 || T < 1 || T > kFewTokens || D < 1 || choice == 1 ||
+      fmoe_host::opt(fmoe_host::kOptFwdAtomicTile) != 0 ||
       fmoe_host::opt(fmoe_host::kOptAtomicOrder) != 0)
     return g;
   g.slices = (D + kWave - 1) / kWave;
@@ -908,7 +923,10 @@ static FewGeom few_geom(int64_t N, int64_t T, int64_t D) {
   shares = std::max<int64_t>(shares, (N + kFewRows - 1) / kFewRows);
   g.rows_per_group = (N + shares - 1) / shares;
   shares = (N + g.rows_per_group - 1) / g.rows_per_group;  // none of them empty
-  g.groups = shares * g.slices;
+  const int64_t groups = shares * g.slices;
+  const int work_bits = N >= 256 * T ? 19 : (groups >= 96 ? 20 : 22);
+  if (choice == 2 || (N >= 4 * T && groups >= 64 && N * D >= (int64_t(1) << work_bits)))
+    g.groups = groups;
   return g;
 }
 
@@ -1191,6 +1209,11 @@ extern "C" int fmoe_combine_fwd(int mode, const void* d_plan, const void* d_indi
 }
 
 extern "C" int64_t fmoe_combine_small_max_rows(void) { return fmoe::kSmallRows; }
+
+extern "C" int64_t fmoe_combine_atomic_few_groups(int64_t num_rows, int64_t num_tokens,
+                                                  int64_t hidden) {
+  return fmoe::few_geom(num_rows, num_tokens, hidden).groups;
+}
 
 extern "C" int fmoe_combine_fwd_small(const int64_t* host_ptrs, const int64_t* host_rows,
                                       int64_t num_experts, const void* d_indices, int idx_dtype,

@@ -24,6 +24,8 @@ enum Opt {
                      // 1 = never, 2 = whenever its limits allow)
   kOptAtomicOrder,   // "fwd_atomic_order": atomic forward's grid order (0 = by size, 1 = row
                      // chunks together, 2 = column-chunk-major)
+  kOptAtomicFew,     // "fwd_atomic_few": atomic forward's few-tokens kernel (0 = by size, 1 = never,
+                     // 2 = whenever the tokens fit)
   kOptCount
 };
 int64_t opt(int o);

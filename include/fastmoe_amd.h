@@ -115,6 +115,9 @@ FMOE_API const char* fmoe_last_error(void);
  *   "fwd_atomic_order" [FMOE_FWD_ATOMIC_ORDER] grid order of the atomic forward: 0 = by size,
  *                                      1 = a row's column chunks side by side, 2 = column-chunk
  *                                      major (all rows' chunk 0, then chunk 1, ...)
+ *   "fwd_atomic_few"  [FMOE_FWD_ATOMIC_FEW] the atomic forward's kernel for few output rows, which
+ *                                      orders a workgroup's rows by token: 0 = by size, 1 = never,
+ *                                      2 = whenever its limits allow
  * fmoe_set_option returns FMOE_EINVAL for an unknown name; *previous (if not NULL) gets the old
  * value.  Not synchronised with launches in flight on other threads.
  */
@@ -256,6 +259,9 @@ FMOE_API int fmoe_invert_scatter_index(const void* d_indices, int idx_dtype, int
  */
 FMOE_API int64_t fmoe_combine_fwd_workspace_bytes(int mode, int64_t num_tokens, int64_t hidden,
                                          int out_dtype);
+/* Workgroups of the few-output-rows kernel that an atomic forward of this size with an fp32 target
+ * takes (option "fwd_atomic_few"), or 0 where it takes the general one. */
+FMOE_API int64_t fmoe_combine_atomic_few_groups(int64_t num_rows, int64_t num_tokens, int64_t hidden);
 FMOE_API int fmoe_combine_fwd(int mode, const void* d_plan, const void* d_indices, int idx_dtype,
                      const void* d_weights, int w_dtype, const int64_t* d_ptr_table,
                      const int64_t* d_offsets, int64_t num_experts, int64_t num_rows,

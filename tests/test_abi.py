@@ -268,3 +268,29 @@ def test_plan_path_reports_the_builder_taken(N, T, auto):
     with _abi.options(plan=3):
         assert lib.fmoe_plan_path(2097152, 1048576, 256) == 1  # beyond the one-launch limits
     assert lib.fmoe_plan_path(-1, 4, 1) == -1 and lib.fmoe_plan_path(4, 0, 1) == -1
+
+
+@pytest.mark.parametrize("N,T,D,groups", [
+    (65536, 128, 1024, 256), (65536, 1000, 1024, 256), (65536, 16, 1024, 256),
+    # too few workgroups for their rows (measured 1.1 to 8 times as slow as the general kernel)
+    (6144, 1024, 64, 0), (8192, 1024, 64, 0), (8192, 1024, 512, 0), (4096, 1024, 2048, 0),
+    (6144, 512, 1024, 0), (6144, 512, 2048, 96), (6145, 512, 1024 * 4, 192),
+    # too little work: below 2^22 from 64 workgroups, 2^20 from 96, 2^19 from 256 rows per token
+    (2048, 256, 2048, 64), (2047, 256, 2048, 0), (512, 16, 2048, 256), (512, 16, 1984, 0),
+    (256, 1, 2048, 256), (256, 1, 2047, 0), (255, 1, 2048, 0),
+    # fewer than 4 rows per token, more tokens than the kernel orders, nothing at all
+    (4095, 1024, 16384, 0), (4096, 1024, 16384, 256), (1 << 20, 1025, 1024, 0), (0, 4, 1024, 0),
+])
+def test_atomic_few_tokens_kernel_by_size(N, T, D, groups):
+    """The atomic forward's few-output-rows kernel is taken only where it has the workgroups and the
+    work to gain by; forced on and off by its option, off by a forced tile or grid order."""
+    few = _abi.lib().fmoe_combine_atomic_few_groups
+    assert few(N, T, D) == groups
+    with _abi.options(fwd_atomic_few=1):
+        assert few(N, T, D) == 0
+    with _abi.options(fwd_atomic_few=2):
+        assert (few(N, T, D) > 0) == (T <= 1024 and N > 0)
+        assert groups == 0 or few(N, T, D) == groups
+    for other in ("fwd_atomic_order", "fwd_atomic_tile"):
+        with _abi.options(**{other: 1}):
+            assert few(N, T, D) == 0

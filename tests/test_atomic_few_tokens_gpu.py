@@ -1,5 +1,6 @@
 """The atomic forward's few-tokens kernel (rows ordered by token within a workgroup): within the
-bound of a reordered fp32 sum of the C oracle's result, at the edges of its rule and shares."""
+bound of a reordered fp32 sum of the C oracle's result, at the edges of its tokens, slices and
+shares."""
 from __future__ import annotations
 
 import numpy as np
@@ -7,25 +8,31 @@ import pytest
 import torch
 
 import fastmoe_amd
+from fastmoe_amd import _abi
 from tests.helpers import abs_sum, oracle_fwd, reorder_tol, to_np, within_one_ulp16
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("T,counts,D,dtype,opts", [
-    (1, [1, 3], 1, torch.float32, {}),
-    (1, [9000], 65, torch.float32, {}),                          # one token, two shares
-    (16, [30, 0, 33], 64, torch.bfloat16, {"bad": True}),        # 63 rows: below 4 per token
-    (16, [31, 0, 33], 64, torch.bfloat16, {"bad": True}),        # 64: the rule's edge
-    (128, [5000, 3192, 1], 100, torch.float32, {"int32": True}),  # shares that end inside an expert
-    (1024, [4096], 200, torch.float32, {}),                      # the most tokens
-    (1025, [4100], 200, torch.float32, {}),                      # one more: k_fwd_atomic
-    (7, [16385], 130, torch.float16, {"w16": True}),             # 3 shares of at most 8192 rows
-    (3, [40, 80], 16400, torch.bfloat16, {}),                    # more slices than workgroups aimed at
+@pytest.mark.parametrize("T,counts,D,dtype,groups,opts", [
+    (1, [1, 3], 1, torch.float32, 1, {}),
+    (1, [9000], 65, torch.float32, 254, {}),                     # one token, 2 slices x 127 shares
+    (16, [30, 0, 33], 64, torch.bfloat16, 1, {"bad": True}),     # 63 rows
+    (16, [31, 0, 33], 64, torch.bfloat16, 1, {"bad": True}),     # 64
+    (128, [5000, 3192, 1], 100, torch.float32, 32, {"int32": True}),  # shares end inside an expert
+    (1024, [4096], 200, torch.float32, 4, {}),                   # the most tokens
+    (1025, [4100], 200, torch.float32, 0, {}),                   # one more: k_fwd_atomic
+    (1024, [8191], 8, torch.float32, 1, {}),                     # one share, a row short of full
+    (7, [16385], 130, torch.float16, 255, {"w16": True}),        # 3 slices x 85 shares
+    (3, [40, 80], 16400, torch.bfloat16, 257, {}),               # more slices than workgroups aimed at
+    (3, [8000, 192], 8257, torch.bfloat16, 130, {}),             # one share of 8192 rows: a full list
+    (3, [8000, 193], 8257, torch.bfloat16, 260, {}),             # one row more: two shares
 ])
 @pytest.mark.parametrize("accumulate", [False, True])
-def test_few_tokens_match_the_oracle(T, counts, D, dtype, opts, accumulate):
+def test_few_tokens_match_the_oracle(T, counts, D, dtype, groups, opts, accumulate, kernel_options):
+    kernel_options(fwd_atomic_few=2)  # whatever the size rule says
+    assert _abi.lib().fmoe_combine_atomic_few_groups(sum(counts), T, D) == groups
     gen = torch.Generator().manual_seed(T + D)
     experts = [torch.randn(n, D, generator=gen).to(dtype) for n in counts]
     N = sum(counts)
@@ -64,6 +71,7 @@ def test_indices_that_change_during_the_call_lose_no_row(dtype):
     takes is open, but each row is added exactly once (rows of ones, unit gates: every column sums
     to N, which fp32 holds exactly)."""
     T, N, D = 128, 65536, 64
+    assert _abi.lib().fmoe_combine_atomic_few_groups(N, T, D) == 128
     routes = [torch.full((N,), t, dtype=dtype, device=DEV) for t in (0, T - 1)]
     idx = routes[0].clone()
     x, w = torch.ones(N, D, device=DEV), torch.ones(N, device=DEV)
