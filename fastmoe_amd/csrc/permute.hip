@@ -328,7 +328,9 @@ __device__ __forceinline__ void copy_row(rsrc_t rs, rsrc_t rd, uint32_t row_byte
 // whose order is the packed order, so a slot's packed row is the number of smaller values: a wave
 // counts them for its slot (N / 64 compares per lane), writes the slot's outputs and copies its
 // row.  Expert e's first row is the number of values below e << 16; those E + 1 counts are spread
-// over the waves of the grid.  Staging reads the N ids once per workgroup from L2, so the gain over
+// over the waves of the grid, which has a wave for every slot or every count, whichever are more (in
+// a graph, N=1, E=4096: 3.2 us, the launches that this replaces 15.4, and 186 with a grid for the
+// slots alone; N=8, E=256: 3.7, 10.0 and 14.8).  Staging reads the N ids once per workgroup from L2, so the gain over
 // rank + place + gather shrinks with N (one MI355X, top-8, E=256, D=7168, bf16, us): N=128 14.1 ->
 // 8.1, N=1024 14.4 -> 9.1, N=2048 16.7 -> 11.1, N=4096 22.4 -> 17.4, where the rows' own copy is
 // most of it.
@@ -591,8 +593,10 @@ static int launch_small(const char* who, const void* d_expert_ids, int id_dtype,
                         void* d_sorted_gates, int32_t* d_slot_pos, int32_t* d_status, void* d_out,
                         hipStream_t s) {
   const int64_t N = T * K;
+  // a wave per slot and per expert bound, whichever are more
+  const int64_t units = std::max(N, E + 1);
   const dim3 grid(std::min<unsigned>(kPermSmallGroups,
-                                     (unsigned)((N + kPermSmallWaves - 1) / kPermSmallWaves)));
+                                     (unsigned)((units + kPermSmallWaves - 1) / kPermSmallWaves)));
   auto launch = [&](auto ti, auto tg, auto vb) {
     using TI = decltype(ti);
     using TG = decltype(tg);

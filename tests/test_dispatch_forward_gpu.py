@@ -19,6 +19,8 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("T,k,E,D,dtype,opts", [
     (1, 1, 1, 1, torch.bfloat16, {}),
     (1, 8, 256, 7168, torch.bfloat16, {}),
+    (1, 1, 4096, 64, torch.bfloat16, {}),                     # most workgroups only count experts
+    (2, 8, 1023, 264, torch.bfloat16, {"bad": True}),
     (5, 3, 4, 100, torch.float16, {"int32": True}),           # 4-byte copies
     (31, 4, 4096, 7, torch.bfloat16, {"bad": True}),          # 2-byte copies, most experts empty
     (512, 8, 256, 264, torch.float32, {"strided": True}),     # 4096 slots: the last one-launch size
