@@ -75,6 +75,7 @@ SIGNATURES: dict[str, tuple] = {
         _c_int,
         [_c_vp, _c_i64, _c_i64, _c_i64, _c_int, _c_vp, _c_int, _c_i64, _c_vp, _c_vp, _c_int, _c_vp],
     ),
+    "fmoe_combine_det_tile": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_int]),
     "fmoe_combine_atomic_few_groups": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "fmoe_combine_small_max_rows": (_c_i64, []),
     "fmoe_combine_fwd_small": (

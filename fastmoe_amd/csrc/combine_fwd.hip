@@ -836,28 +836,49 @@ constexpr unsigned lds_for_groups(int groups) { return (160u << 10) / 1280 / gro
 //   fp32: T=4096, D=16384, k=8  427.4 -> 404.0 (433.4); k=4  227.7 -> 215.7 (224.9)
 // With 2 workgroups T=8192, D=4096, k=6 takes 81.7 us and T=4096, D=8192, k=8 98.1; r < 2.5 loses
 // under every bound (T=8192, D=4096, k=2: 31.9, 36.7 with 3 workgroups).
+//
+// Few wave units.  A wider tile makes fewer of them, and below 1280 (U = 4; 1024 for U = 2), five or
+// four to a CU, the waves missing cost more than the tile gains, at every size of the rows: those
+// calls keep the tile by D and r (narrow_det_tile), where U = 4 gives way to U = 2 below 512 wave
+// units.  The kernel alone, bf16, us, the tile above / the tile by D and r, wave units of the former:
+//   T=256, D=2048, k=8:   256,  7.0 /  4.6     T=512, D=2048, k=8:    512,  7.4 /  5.8
+//   T=256, D=1536, k=8:   512,  5.0 /  4.4     T=512, D=4096, k=4:   1024,  6.0 /  5.4
+//   T=1024, D=4096, k=8: 2048, 13.7 / 14.1     T=1024, D=3072, k=4:  2048,  7.4 /  7.6
+//   N=131072: T=64, D=1024: 64, 506 / 362      T=16, D=4096: 64, 1961 / 3169 with U = 4
+static DetTile narrow_det_tile(int64_t N, int64_t T, int64_t D, int V) {
+  DetTile c{pick_u(D, V), 0, 0};
+  c.R = c.U >= 4 ? 4 : 8;
+  if (2 * N < 7 * T) {
+    if (c.U >= 2) c.R = 4;
+  } else if (c.U == 4) {
+    const int64_t CW = (int64_t)kWave * V * 4;
+    if (T * ((D + CW - 1) / CW) < 512) c = {2, 4, 0};
+  } else if (N >= 7 * T && c.U == 2) {
+    c = {1, 8, 0};
+  }
+  return c;
+}
+
 static DetTile pick_det_tile(int64_t N, int64_t T, int64_t D, int64_t x_bytes, int V) {
   DetTile c{pick_u(D, V), 0, 0};
   c.R = c.U >= 4 ? 4 : 8;
   if (fmoe_host::opt(fmoe_host::kOptFwdDetU) != 0 || N == 0) return c;  // U forced: keep R by U
   const int64_t bytes = N * D * x_bytes;
   if (2 * N <= 3 * T && D >= (int64_t)kWave * V * 4) return {4, 2, 0};  // r <= 1.5
-  if (2 * N < 5 * T) {                                                  // r < 2.5
-    if (c.U >= 2) c.R = 4;
-    return c;
-  }
+  if (2 * N < 5 * T) return narrow_det_tile(N, T, D, V);                // r < 2.5
   if (D < (int64_t)kWave * V * 2) return c;  // less than a chunk of 2 vectors per lane
   if (bytes >= (int64_t(256) << 20)) {
-    if (2 * N < 7 * T) return {2, 4, lds_for_groups(4)};
-    if (N >= 7 * T && bytes >= (int64_t(768) << 20)) return {2, 4, lds_for_groups(2)};
-    return {2, 4, lds_for_groups(3)};
+    const bool two = N >= 7 * T && bytes >= (int64_t(768) << 20);
+    c = {2, 4, lds_for_groups(2 * N < 7 * T ? 4 : (two ? 2 : 3))};
+  } else if (2 * N < 7 * T) {  // r < 3.5
+    return narrow_det_tile(N, T, D, V);
+  } else if (D >= (int64_t)kWave * V * 4) {
+    c = {4, 2, 0};
+  } else {
+    c = {2, 4, 0};
   }
-  if (2 * N < 7 * T) {  // 2.5 <= r < 3.5
-    if (c.U >= 2) c.R = 4;
-    return c;
-  }
-  if (D >= (int64_t)kWave * V * 4) return {4, 2, 0};
-  return {2, 4, 0};
+  const int64_t CW = (int64_t)kWave * V * c.U;
+  return T * ((D + CW - 1) / CW) < (c.U == 4 ? 1280 : 1024) ? narrow_det_tile(N, T, D, V) : c;
 }
 
 // Tile shapes (U vectors per lane per row, R rows per batch).  The "fwd_tile" option <U><R> (e.g.
@@ -1206,6 +1227,18 @@ extern "C" int fmoe_combine_fwd(int mode, const void* d_plan, const void* d_indi
                                        a.s)
              : launch_acc_pass<f16_t>(false, acc, d_out, out_row_stride, hidden, num_tokens, 1,
                                       a.s);
+}
+
+extern "C" int64_t fmoe_combine_det_tile(int64_t num_rows, int64_t num_tokens, int64_t hidden,
+                                         int x_dtype) {
+  if (num_rows < 1 || num_tokens < 1 || hidden < 1 || !fmoe_host::is_float_dtype(x_dtype)) return -1;
+  const int eb = fmoe_host::dtype_bytes(x_dtype);
+  if (hidden % (16 / eb) != 0) return 0;
+  const fmoe::DetTile c = fmoe::pick_det_tile(num_rows, num_tokens, hidden, eb, 16 / eb);
+  int groups = 0;
+  for (int g = 2; g <= 4; ++g)
+    if (c.lds != 0 && c.lds == fmoe::lds_for_groups(g)) groups = g;
+  return groups * 100 + c.U * 10 + c.R;
 }
 
 extern "C" int64_t fmoe_combine_small_max_rows(void) { return fmoe::kSmallRows; }

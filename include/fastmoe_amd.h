@@ -259,6 +259,11 @@ FMOE_API int fmoe_invert_scatter_index(const void* d_indices, int idx_dtype, int
  */
 FMOE_API int64_t fmoe_combine_fwd_workspace_bytes(int mode, int64_t num_tokens, int64_t hidden,
                                          int out_dtype);
+/* Tile that the deterministic forward and fmoe_permute_backward (num_rows = T * top_k) choose for
+ * rows of 16-byte vectors, by size: U * 10 + R (16-byte vectors per lane per row, rows per batch),
+ * plus 100 times the workgroups that may be resident on a CU where that is bounded; 0 for rows that
+ * no 16-byte vector divides, -1 for bad sizes. */
+FMOE_API int64_t fmoe_combine_det_tile(int64_t num_rows, int64_t num_tokens, int64_t hidden, int x_dtype);
 /* Workgroups of the few-output-rows kernel that an atomic forward of this size with an fp32 target
  * takes (option "fwd_atomic_few"), or 0 where it takes the general one. */
 FMOE_API int64_t fmoe_combine_atomic_few_groups(int64_t num_rows, int64_t num_tokens, int64_t hidden);

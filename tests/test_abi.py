@@ -294,3 +294,26 @@ def test_atomic_few_tokens_kernel_by_size(N, T, D, groups):
     for other in ("fwd_atomic_order", "fwd_atomic_tile"):
         with _abi.options(**{other: 1}):
             assert few(N, T, D) == 0
+
+
+@pytest.mark.parametrize("N,T,D,dtype,tile", [
+    # few wave units keep the tile by D and rows per token (the wide ones measured up to 1.5 times
+    # as slow there)
+    (2048, 256, 2048, "BF16", 18), (4096, 512, 2048, "BF16", 18), (2048, 256, 1536, "BF16", 18),
+    (512, 64, 7168, "BF16", 18), (2048, 512, 4096, "BF16", 44), (2048, 256, 1024, "F32", 18),
+    (2044, 511, 1536, "BF16", 18), (131072, 64, 1024, "BF16", 18), (32768, 4, 7168, "BF16", 18),
+    (131072, 16, 4096, "BF16", 24), (131072, 255, 4096, "BF16", 24), (131072, 256, 4096, "BF16", 224),
+    (131072, 511, 2048, "BF16", 18), (131072, 512, 2048, "BF16", 324), (2048, 512, 1536, "BF16", 24),
+    (2556, 639, 4096, "BF16", 44), (2560, 640, 4096, "BF16", 42), (8192, 1024, 4096, "BF16", 42),
+    # rows per token: up to 1.5, below 2.5, below 3.5
+    (768, 512, 2048, "BF16", 42), (1279, 512, 4096, "BF16", 44), (3584, 1024, 2048, "BF16", 28),
+    (3583, 1024, 2048, "BF16", 24), (3583, 1024, 1024, "BF16", 18),
+    # rows from 256 MiB: by rows per token and size, 4, 3 or 2 workgroups to a CU
+    (16384, 5462, 8192, "BF16", 424), (16384, 4097, 8192, "BF16", 324), (16383, 4680, 8192, "BF16", 42), (16383, 4681, 8192, "BF16", 44),
+    (32768, 2048, 12288, "BF16", 224), (32768, 4682, 6144, "F32", 324), (32768, 4681, 6148, "F32", 224),
+    # less than a chunk of 2 vectors per lane; element-wise; nothing
+    (2048, 512, 1000, "BF16", 18), (2048, 512, 1001, "BF16", 0), (0, 512, 1024, "BF16", -1),
+    (8, 4, 1024, "I64", -1),
+])
+def test_deterministic_tile_by_size(N, T, D, dtype, tile):
+    assert _abi.lib().fmoe_combine_det_tile(N, T, D, getattr(_abi, dtype)) == tile

@@ -13,6 +13,10 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("T,D,N,dtype", [
+    (512, 2048, 4096, torch.bfloat16),       # few wave units: the tile by D and r
+    (639, 4096, 2556, torch.bfloat16),       # 1278 of 4 vectors: still
+    (640, 4096, 2560, torch.bfloat16),       # 1280
+    (511, 1536, 2044, torch.bfloat16),       # 1022 of 2 vectors
     (512, 2048, 768, torch.bfloat16),        # r = 1.5
     (512, 2048, 1279, torch.bfloat16),       # below 2.5
     (512, 2056, 1280, torch.bfloat16),       # 2.5, small rows
