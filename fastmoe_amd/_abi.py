@@ -17,7 +17,8 @@ ABI_VERSION = 2
 
 # enum fmoe_dtype / fmoe_mode / fmoe_status (include/fastmoe_amd.h)
 F32, BF16, F16, I64, I32 = 0, 1, 2, 3, 4
-MODE_DET, MODE_ATOMIC, MODE_ATOMIC_PACKED = 0, 1, 2
+MODE_DET, MODE_ATOMIC, MODE_ATOMIC_PACKED, MODE_DET_STEP = 0, 1, 2, 3
+STREAM_OUT_BYTES = 96 << 20  # FMOE_STREAM_OUT_BYTES
 OK, EINVAL, EHIP, ERANGE = 0, -1, -2, -3
 
 _c_i64 = ctypes.c_int64

@@ -723,6 +723,7 @@ static int grid_for(int64_t units, const char* who, unsigned* blocks) {
 
 struct FwdArgs {
   int mode;
+  bool step;  // FMOE_MODE_DET_STEP
   const int32_t* status;
   const int32_t* row_ptr;
   const Rec* rec;
@@ -740,24 +741,29 @@ struct FwdArgs {
   hipStream_t s;
 };
 
-// Output bytes from which the deterministic forward stores its output non-temporally.  Stored with
-// the temporal policy (FMOE_OUT_CPOL), the output stays dirty in the 256 MB Infinity Cache: the
-// forward itself is up to 5 % shorter, but its lines are written back during the kernels that
-// follow, which loses more once the output is a large part of that cache.  Measured on one MI355X
-// with three sets of buffers in turn (bf16, us per call; temporal / non-temporal):
-//   T, D, k (output)             forward          forward + backward
-//   8192, 4096, 6 (64 MiB)       77.6 /  81.2     246.0 / 228.6
-//   2048, 16384, 8 (64 MiB)     100.0 / 101.6     313.7 / 297.5
-//   3072, 16384, 8 (96 MiB)     164.2 / 159.6     469.4 / 451.7
-//   4096, 16384, 8 (128 MiB)    217.2 / 212.2     635.9 / 613.4
-//   16384, 4096, 6 (128 MiB)    167.1 / 160.0     483.8 / 463.8
-//   6144, 16384, 8 (192 MiB)    324.4 / 319.7     930.4 / 922.9
-//   32768, 16384, 2 (1 GiB)     520.5 / 523.2    1677.7 / 1623.8
-// The line lies where the forward alone gains too; below it a program that only runs forwards
-// keeps the shorter one.  An accumulating call has just read its output and the caller has just
+// Whether the deterministic forward stores its output non-temporally.  Stored with the temporal
+// policy (FMOE_OUT_CPOL), the output stays dirty in the 256 MB Infinity Cache: the forward itself is
+// shorter if the output's lines are still there from the call before (a loop that writes the same
+// buffer), but they are written back during the kernels that follow, which loses more once the output
+// is a large part of that cache.  Time non-temporal / temporal, bf16 but for the last row (one MI355X,
+// three sets of inputs; the forward alone into one buffer | into three in turn | with its backward):
+//   T, D (output)              top-1                top-3                top-8
+//   12288, 4096 (96 MiB)       1.11 | 1.03 | 0.99   1.07 | 0.97 | 0.94   1.01 | 0.94 | 0.95
+//   16384, 4096 (128 MiB)      1.11 | 0.98 | 0.92   1.05 | 0.97 | 0.95   1.01 | 0.96 | 0.96
+//   4096, 16384 (128 MiB)      1.13 | 0.97 | 0.97   1.06 | 0.97 | 0.94   1.02 | 0.99 | 0.96
+//   16384, 7168 (224 MiB)      1.17 | 1.00 | 0.92   1.08 | 0.99 | 0.93   1.01 | 1.00 | 0.94
+//   16384, 12288 (384 MiB)     1.00 | 1.00 | 0.99   1.00 | 1.01 | 0.95
+//   fp32 8192, 8192 (256 MiB)  1.15 | 0.98 | 0.95   1.07 | 0.99 | 0.91   1.06 | 1.01 | 0.93
+// So a forward whose backward follows streams from 96 MiB, and one alone only from 7 rows per token,
+// where it gains as much in a program that goes on to other buffers as it loses in one that does not.
+// Steps below that line (2048, 16384, top-8, 64 MiB: 313.7 -> 297.5 us) stay temporal with the
+// forwards.  An accumulating call has just read its output and the caller has just
 // written it, so its lines are in the cache: fp32, 256 MiB, zero-fill + call 291.6 us temporal,
 // 316.9 us non-temporal; it stays temporal.
-constexpr int64_t kOutStreamBytes = int64_t(96) << 20;
+static int streams_out(const FwdArgs& a, int64_t elem_bytes) {
+  return !a.accumulate && a.T * a.D * elem_bytes >= FMOE_STREAM_OUT_BYTES &&
+         (a.step || a.N >= 7 * a.T);
+}
 
 template <typename TX, typename TO, int V, int U, int RB>
 static int launch_fwd_k(const FwdArgs& a, int64_t chunks) {
@@ -769,7 +775,7 @@ static int launch_fwd_k(const FwdArgs& a, int64_t chunks) {
     hipLaunchKernelGGL((k_fwd_det<TX, TO, V, U, RB>), dim3(blocks), dim3(kGroup), a.lds, a.s, a.status,
                        a.row_ptr, a.rec, static_cast<TO*>(a.out), a.out_stride, (uint32_t)a.D,
                        (uint32_t)a.T, (uint32_t)chunks, a.accumulate,
-                       !a.accumulate && a.T * a.D * (int64_t)sizeof(TO) >= kOutStreamBytes);
+                       streams_out(a, sizeof(TO)));
     return fmoe_host::check_launch("fmoe_combine_fwd(det)");
   }
   if constexpr (V == 1 && sizeof(TO) == 2) {
@@ -1006,7 +1012,7 @@ struct SlotsBwdArgs {
   unsigned lds;  // DetTile
 };
 
-// grad_x is streamed from a smaller size than the forward's output (kOutStreamBytes): a backward is
+// grad_x is streamed from a smaller size than the forward's output (streams_out): a backward is
 // always followed by more passes over as much data, which pay for the lines left in the cache.
 // Permutation forward + backward, three sets of buffers in turn, bf16, temporal / non-temporal:
 // T=8192, D=4096, top-6 and T=4096, D=8192, top-6 (64 MiB) 180.9 / 165.9 and 182.0 / 164.8 us;
@@ -1132,6 +1138,8 @@ extern "C" int fmoe_combine_fwd(int mode, const void* d_plan, const void* d_indi
                                 void* d_workspace, int64_t workspace_bytes, void* stream) {
   using namespace fmoe;
   fmoe_host::clear_error();
+  const bool step = mode == FMOE_MODE_DET_STEP;
+  if (step) mode = FMOE_MODE_DET;
   FMOE_REQUIRE(mode == FMOE_MODE_DET || mode == FMOE_MODE_ATOMIC || mode == FMOE_MODE_ATOMIC_PACKED,
                "fmoe_combine_fwd: bad mode %d", mode);
   FMOE_REQUIRE(num_rows >= 0 && num_tokens >= 1 && hidden >= 1,
@@ -1153,6 +1161,7 @@ extern "C" int fmoe_combine_fwd(int mode, const void* d_plan, const void* d_indi
   }
   FwdArgs a{};
   a.mode = mode;
+  a.step = step;
   a.N = num_rows;
   a.T = num_tokens;
   a.D = hidden;

@@ -129,7 +129,7 @@ constexpr int kCPolCached = 0;  // default policy: keep in L2 / Infinity Cache (
 #define FMOE_X_CPOL 2    // expert-row loads (read once): non-temporal
 #endif
 #ifndef FMOE_OUT_CPOL
-#define FMOE_OUT_CPOL 16 // forward output stores below kOutStreamBytes: SC1 (device scope), temporal
+#define FMOE_OUT_CPOL 16 // forward output stores unless streams_out: SC1 (device scope), temporal
 #endif
 #ifndef FMOE_BWD_WAVES
 #define FMOE_BWD_WAVES 8 // waves per token workgroup of the backward (one row each at top-8)

@@ -537,7 +537,7 @@ def _launch_fwd_raw(mode: int, plan: Optional[int], idx: Optional[torch.Tensor],
         # the fp32 accumulator of a 16-bit output (fmoe_combine_fwd_workspace_bytes)
         ws_bytes = lib.fmoe_combine_fwd_workspace_bytes(mode, T, D, out_code)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    name = "fwd_det" if mode == _abi.MODE_DET else "fwd_atomic"
+    name = "fwd_det" if mode in (_abi.MODE_DET, _abi.MODE_DET_STEP) else "fwd_atomic"
     with _on_device(dev), _span(name):
         rc = lib.fmoe_combine_fwd(
             mode, plan,
@@ -701,6 +701,8 @@ def _combine_forward(ctx, mode: Optional[str], validate: Optional[bool], indices
             if _validate_default(validate):
                 _check_plan_status(meta.plan_tensor(), T)
         out = torch.empty(shape, dtype=dtype, device=dev)
+        if ctx is not None and T * hidden * _ELEM_BYTES[dtype] >= _abi.STREAM_OUT_BYTES:
+            code = _abi.MODE_DET_STEP  # a backward follows
         _launch_fwd_raw(code, meta.plan, None, None, meta.ptr_table, meta.offsets, ex.num, rows,
                         dtype, out, accumulate=False)
     else:

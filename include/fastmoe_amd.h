@@ -75,8 +75,13 @@ enum fmoe_mode {
   /* As FMOE_MODE_ATOMIC, but a bf16/f16 `out` takes gfx950's packed 16-bit atomics
      (global_atomic_pk_add_bf16 / _f16) directly: no workspace, half the atomic requests, and a
      rounding to 16 bits at every add (the reference Triton kernel's behaviour with a bf16 out). */
-  FMOE_MODE_ATOMIC_PACKED = 2
+  FMOE_MODE_ATOMIC_PACKED = 2,
+  /* FMOE_MODE_DET, bit for bit, for a forward that its backward follows: an overwritten `out` of
+     FMOE_STREAM_OUT_BYTES or more is stored past the caches, which pays over the whole step.
+     FMOE_MODE_DET does so only from 7 rows per token. */
+  FMOE_MODE_DET_STEP = 3
 };
+#define FMOE_STREAM_OUT_BYTES (96ll << 20)
 
 enum fmoe_status {
   FMOE_OK = 0,
@@ -242,7 +247,7 @@ FMOE_API int fmoe_invert_scatter_index(const void* d_indices, int idx_dtype, int
  * Forward combine (replaces _launch_grouped_kernel + _grouped_weighted_scatter_add_kernel,
  * src/fastmoe/kernels/ops.py:277-310 and :57-194).
  *
- * mode == FMOE_MODE_DET     : reads the plan (d_plan from fmoe_build_plan on the same inputs);
+ * mode == FMOE_MODE_DET[_STEP] : reads the plan (d_plan from fmoe_build_plan on the same inputs);
  *                             d_indices/d_weights/d_ptr_table/d_offsets may be NULL.
  * mode == FMOE_MODE_ATOMIC[_PACKED] : reads d_indices/d_weights/d_ptr_table/d_offsets; d_plan may
  *                             be NULL.

@@ -41,6 +41,13 @@ def test_no_other_symbols_exported():
     assert not [n for n in exported if n.startswith("_ZN4fmoe")]
 
 
+def test_step_mode_and_its_output_size_are_the_headers():
+    text = HEADER.read_text()
+    assert f"FMOE_MODE_DET_STEP = {_abi.MODE_DET_STEP}\n" in text
+    assert f"#define FMOE_STREAM_OUT_BYTES ({_abi.STREAM_OUT_BYTES >> 20}ll << 20)" in text
+    assert _abi.lib().fmoe_combine_fwd_workspace_bytes(_abi.MODE_DET_STEP, 4, 8, _abi.BF16) == 0
+
+
 def test_plan_layout_functions():
     lib = _abi.lib()
     N, T = 32768, 4096

@@ -80,7 +80,7 @@ class FakeLib:
 
     def fmoe_combine_fwd(self, mode, plan, idx, idt, w, wdt, ptr_table, offsets, E, N, T, D, xdt,
                          out, odt, ostride, acc, ws, ws_bytes, stream):
-        if mode == _abi.MODE_DET:
+        if mode in (_abi.MODE_DET, _abi.MODE_DET_STEP):
             assert isinstance(plan, int)
         else:
             assert isinstance(idx, int) and isinstance(w, int)
@@ -160,6 +160,20 @@ def test_autograd_forward_and_backward_calls(fake):
     assert fake.calls[2] == ("bwd", 8, 4, 16, _abi.BF16, 16, True, True, _abi.F32)
     assert grads[0].shape == (N,) and grads[0].dtype == torch.float32
     assert [g.shape[0] for g in grads[1:]] == [3, 0, 5]
+
+
+def test_large_output_of_a_recorded_forward_is_marked_as_a_step(fake):
+    """Only a forward that records a backward, and only from the size at which the library streams
+    the output."""
+    D, T = 4096, _abi.STREAM_OUT_BYTES // (4096 * 2)
+    xs = _experts(sizes=(3, 0, 5), D=D)
+    idx = torch.randint(0, 4, (8,))
+    for t, w, mode in ((T, torch.rand(8, requires_grad=True), _abi.MODE_DET_STEP),
+                       (T - 1, torch.rand(8, requires_grad=True), _abi.MODE_DET),
+                       (T, torch.rand(8), _abi.MODE_DET)):
+        fake.calls.clear()
+        fastmoe_amd.grouped_weighted_scatter_add(xs, idx, w, (t, D))
+        assert [c[:2] for c in fake.calls if c[0] == "fwd"] == [("fwd", mode)]
 
 
 class _Timer:

@@ -1,5 +1,5 @@
 """The deterministic forward's non-temporal output stores: outputs of 96 MiB or more that the call
-overwrites.  Sizes on both sides of that line, vector and element-wise columns, padded rows and an
+overwrites, in a step or from 7 rows per token.  Sizes on both sides of that line, vector and element-wise columns, padded rows and an
 accumulating call (which never takes them), bit for bit against the C oracle."""
 from __future__ import annotations
 
@@ -22,7 +22,8 @@ DEV = "cuda:0"
     (12300, 4097, torch.float16, 0, False),    # element-wise columns, a partial last chunk
     (6145, 4104, torch.float32, 0, False),     # vectors, a partial last chunk
 ])
-def test_large_outputs_match_the_oracle(T, D, dtype, pad, accumulate):
+@pytest.mark.parametrize("mode", [_abi.MODE_DET_STEP, _abi.MODE_DET])  # streamed, not
+def test_large_outputs_match_the_oracle(T, D, dtype, pad, accumulate, mode):
     gen = torch.Generator().manual_seed(5)
     counts = [120, 0, 77, 103]
     experts = [torch.randn(n, D, generator=gen).to(dtype) for n in counts]
@@ -35,7 +36,19 @@ def test_large_outputs_match_the_oracle(T, D, dtype, pad, accumulate):
                                                w.to(DEV), T)
     full = torch.full((T, D + pad), 0.0 if accumulate else 7.0, dtype=dtype, device=DEV)
     out = full[:, :D]
-    ops._launch_fwd(meta, _abi.MODE_DET, plan, None, None, out, accumulate=accumulate)
+    ops._launch_fwd(meta, mode, plan, None, None, out, accumulate=accumulate)
     assert np.array_equal(bits(out), want.view(np.uint32) if dtype == torch.float32 else want)
     if pad:
         assert bool((full[:, D:] == 7.0).all())
+
+
+@pytest.mark.parametrize("rows", [7, 6])  # per token: streamed by the forward alone, not
+def test_forward_alone_and_in_a_step_agree(rows):
+    T, D = 12288, 4096
+    gen = torch.Generator(device=DEV).manual_seed(6)
+    x = torch.randn(T * rows, D, generator=gen, device=DEV).bfloat16()
+    idx = torch.randint(0, T, (T * rows,), generator=gen, device=DEV)
+    w = torch.rand(T * rows, generator=gen, device=DEV)
+    alone = ops.weighted_scatter_add(x, idx, w, (T, D))
+    step = ops.weighted_scatter_add(x, idx, w.clone().requires_grad_(True), (T, D))
+    assert step.requires_grad and torch.equal(alone, step.detach())
