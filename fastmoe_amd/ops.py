@@ -566,24 +566,36 @@ def _launch_fwd(meta: GroupedMetadata, mode: int, plan: Optional[torch.Tensor],
 # step is two launches instead of four (metadata + plan, forward, grad_w pass, grad_X pass), and a
 # forward saves the plan's dependent launch.  Each forward wave scans the token id of every row, so
 # the cost grows with T * N: calls with T * N <= _SMALL_ALWAYS take it, and up to _SMALL_SCAN_LIMIT
-# those of at most _SMALL_TOKENS tokens (the waves of its grid).  Its backward writes grad_X between
-# its reads, which the planned passes keep apart, so a call that records a backward takes it beyond
-# _SMALL_ALWAYS only while its rows are at most _SMALL_STEP_BYTES.  Launches in graphs on one MI355X, bf16, forward + backward in us, planned -> small:
-#   T=64, D=7168, top-8     11.5 + 9.6 ->  6.0 + 7.8     T=1024, D=1024, top-4   11.2 + 7.0 -> 10.0 + 6.0
-#   T=256, D=7168, top-8   14.6 + 12.4 ->  9.7 + 14.6    T=256, D=16384, top-8  19.0 + 24.4 -> 15.7 + 31.6
-#   T=512, D=4096, top-6   13.6 + 11.7 -> 10.1 + 12.6    T=512, D=7168, top-8   18.1 + 22.6 -> 17.2 + 27.2
-# and past the scan's limit T=4096, D=2048, top-1: 13.8 -> 15.5 forward.
+# those of at most _SMALL_TOKENS tokens (the waves of its grid) whose rows are small enough:
+# * a forward alone while T * N times the bytes of its rows is at most _SMALL_SCAN_BYTES, beyond which
+#   the scans cost more than the plan;
+# * a call that records a backward while its rows are at most _SMALL_STEP_BYTES and _SMALL_STEP_ROWS,
+#   or _SMALL_STEP_ANY bytes: its backward writes grad_X between its reads, which the planned passes
+#   keep apart.
+# Launches in graphs on one MI355X, three sets of buffers in turn, us, planned -> small:
+#   forward, bf16                                  forward + backward, bf16
+#   T=64, D=7168, top-8          10.4 ->  5.9      T=64, D=7168, top-8      20.1 -> 14.6
+#   T=256, D=7168, top-8         15.9 -> 11.7      T=256, D=7168, top-8     29.9 -> 29.2
+#   T=512, D=7168, top-8         20.4 -> 19.3      T=512, D=4096, top-6     28.3 -> 28.6
+#   T=1024, D=7168, top-4        21.8 -> 22.4      T=512, D=1024, top-8     19.0 -> 18.1
+#   T=1024, D=16384, top-4       38.6 -> 39.7      T=512, D=2048, top-8     22.6 -> 24.8
+#   fp32: T=2048, D=16384, top-1 54.8 -> 58.8      T=256, D=4096, top-16    32.6 -> 36.1
+# and past the scan's limit T=4096, D=2048, top-1: 16.1 -> 17.0 forward.
 _SMALL_MAX_EXPERTS = 256
 _SMALL_ALWAYS = 1 << 17
 _SMALL_SCAN_LIMIT = 1 << 22
 _SMALL_TOKENS = 4096
+_SMALL_SCAN_BYTES = 1 << 48
 _SMALL_STEP_BYTES = 32 << 20
+_SMALL_STEP_ROWS = 3072
+_SMALL_STEP_ANY = 8 << 20
 _SMALL_MAX_ROWS: list = []
 
 
-def _use_small(rows: int, num_tokens: int, num_experts: int, step_bytes: int = 0) -> bool:
+def _use_small(rows: int, num_tokens: int, num_experts: int, step_bytes: int = 0,
+               fwd_bytes: int = 0) -> bool:
     """Whether a deterministic call takes the small path; ``step_bytes``: the bytes of its expert
-    rows if it records a backward, else 0."""
+    rows if it records a backward, ``fwd_bytes``: if it does not."""
     choice = _abi.option("small")
     if choice == 1 or _abi.option("plan") != 0 or num_experts > _SMALL_MAX_EXPERTS or rows < 1:
         return False
@@ -592,9 +604,12 @@ def _use_small(rows: int, num_tokens: int, num_experts: int, step_bytes: int = 0
     if rows > _SMALL_MAX_ROWS[0]:
         return False
     scan = rows * num_tokens
-    return (choice == 2 or scan <= _SMALL_ALWAYS
-            or (scan <= _SMALL_SCAN_LIMIT and num_tokens <= _SMALL_TOKENS
-                and step_bytes <= _SMALL_STEP_BYTES))
+    if choice == 2 or scan <= _SMALL_ALWAYS:
+        return True
+    if scan > _SMALL_SCAN_LIMIT or num_tokens > _SMALL_TOKENS:
+        return False
+    return (scan * fwd_bytes <= _SMALL_SCAN_BYTES and step_bytes <= _SMALL_STEP_BYTES
+            and (rows <= _SMALL_STEP_ROWS or step_bytes <= _SMALL_STEP_ANY))
 
 
 def _launch_fwd_small(tables, num_experts: int, idx: torch.Tensor, w: torch.Tensor,
@@ -634,7 +649,8 @@ def _launch_grouped_kernel(expert_tensors, indices, weights, out, metadata=None,
         # ``out``; a validating call takes the planned path, which raises before any forward
         # launch, so ``out`` is left untouched when it raises.
         if (code == _abi.MODE_DET and not _validate_default(validate)
-                and _use_small(ex.rows, T, ex.num)):
+                and _use_small(ex.rows, T, ex.num,
+                               fwd_bytes=ex.rows * ex.hidden * _ELEM_BYTES[ex.dtype])):
             _check_out(out, None, ex.hidden, ex.device)
             _launch_fwd_small(ex.host_tables(), ex.num, idx, w, ex.dtype, out, accumulate=True)
             return out
@@ -681,8 +697,9 @@ def _combine_forward(ctx, mode: Optional[str], validate: Optional[bool], indices
         meta = _RawMeta(ex)
         _run_metadata(ex, meta)
         out = torch.zeros(shape, dtype=dtype, device=dev)
-    elif code == _abi.MODE_DET and _use_small(
-            rows, T, ex.num, rows * hidden * _ELEM_BYTES[dtype] if ctx is not None else 0):
+    elif code == _abi.MODE_DET and _use_small(rows, T, ex.num, *(
+            (rows * hidden * _ELEM_BYTES[dtype], 0) if ctx is not None
+            else (0, rows * hidden * _ELEM_BYTES[dtype]))):
         # one launch, no plan; the backward is one launch too
         small = ex.host_tables()
         out = torch.empty(shape, dtype=dtype, device=dev)

@@ -378,10 +378,32 @@ def test_small_path_forward_only(fake_small):
     assert [c[0] for c in fake_small.calls] == ["fwd_small"]
 
 
+@pytest.mark.parametrize("rows,T,D,records,small", [
+    # a forward alone: T * N times the rows' bytes up to 2^48
+    (4096, 512, 7168, False, True), (4096, 1024, 8192, False, True), (4096, 1024, 8200, False, False),
+    (2048, 2048, 16384, False, True), (4096, 1024, 16384, False, False),
+    # with its backward: rows up to 32 MiB and 3072 of them, or 8 MiB
+    (2048, 256, 8192, True, True), (2048, 256, 8200, True, False), (3072, 512, 5461, True, True),
+    (3073, 512, 5456, True, False), (4096, 512, 1024, True, True), (4096, 512, 1032, True, False),
+    # small scans whatever the rows
+    (4096, 32, 16384, True, True), (4096, 33, 16384, True, False),
+])
+def test_small_path_by_scan_and_row_bytes(fake_small, rows, T, D, records, small):
+    x = torch.empty(rows, D, dtype=torch.bfloat16, requires_grad=records)
+    fastmoe_amd.weighted_scatter_add(x, torch.zeros(rows, dtype=torch.long), torch.rand(rows), (T, D))
+    assert fake_small.calls[-1][0] == ("fwd_small" if small else "fwd")
+    if not records:  # the in-place call follows the forward alone
+        fake_small.calls.clear()
+        out = torch.empty(T, D, dtype=torch.bfloat16)
+        fastmoe_amd.weighted_scatter_add(x, torch.zeros(rows, dtype=torch.long), torch.rand(rows),
+                                         (T, D), out)
+        assert fake_small.calls[-1][0] == ("fwd_small" if small else "fwd")
+
+
 @pytest.mark.parametrize("case", ["off", "plan_forced", "atomic", "experts", "rows", "scan"])
 def test_small_path_not_taken(fake_small, case):
     """The small path stays out of forced plans, atomic modes, more than 256 experts or 4096 rows,
-    and (by default) calls whose forward scan T * N exceeds 2^17."""
+    and (by default) calls whose forward scan T * N exceeds 2^17 with more than 4096 tokens."""
     sizes, T, opts, mode = (3, 0, 5), 4, {}, None
     if case == "off":
         opts = {"small": 1}
