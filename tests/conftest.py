@@ -46,3 +46,19 @@ def kernel_options():
     yield set_options
     for k, v in saved.items():
         _abi.set_option(k, v)
+
+
+@pytest.fixture
+def library_calls(monkeypatch):
+    """The entry points called so far, in order: a test that means one path says so."""
+    from fastmoe_amd import _abi
+
+    calls = []
+    check = _abi.check
+
+    def record(rc, what):
+        calls.append(what)
+        return check(rc, what)
+
+    monkeypatch.setattr(_abi, "check", record)
+    return calls

@@ -63,6 +63,33 @@ def test_permutation_matches_the_oracle(T, k, E, D, dtype, opts):
             fastmoe_amd.permute_tokens(xd, ids.to(DEV), gates.to(DEV), E, validate=True)
 
 
+@pytest.mark.parametrize("T,k,E,bad", [(1, 1, 1, False), (37, 3, 8, True), (512, 8, 256, True),
+                                       (300, 4, 3000, False), (1000, 4, 1024, True)])
+def test_separate_calls_give_the_one_launch_outputs(T, k, E, bad):
+    """fmoe_permute_build and fmoe_permute_gather at sizes that fmoe_permute takes in one launch."""
+    gen = torch.Generator().manual_seed(T)
+    ids = torch.randint(0, E, (T, k), generator=gen)
+    if bad:
+        ids.view(-1)[::5] = E
+    ids, gates = ids.to(DEV), torch.rand(T, k, generator=gen).to(DEV)
+    x = torch.randn(T, 40, generator=gen).to(DEV)
+    p = fastmoe_amd.permute_tokens(x, ids, gates, E)
+    lib, N, stream = _abi.lib(), T * k, torch.cuda.current_stream().cuda_stream
+    got = [torch.full_like(t, 7) for t in p]
+    rows, counts, rev, sorted_gates, offsets, slot_pos = got
+    status = torch.empty(1, dtype=torch.int32, device=DEV)
+    ws = torch.empty(lib.fmoe_permute_workspace_bytes(N, E), dtype=torch.uint8, device=DEV)
+    _abi.check(lib.fmoe_permute_build(
+        ids.data_ptr(), _abi.I64, gates.data_ptr(), _abi.F32, T, k, E, counts.data_ptr(),
+        offsets.data_ptr(), rev.data_ptr(), sorted_gates.data_ptr(), slot_pos.data_ptr(),
+        status.data_ptr(), ws.data_ptr(), stream), "fmoe_permute_build")
+    _abi.check(lib.fmoe_permute_gather(slot_pos.data_ptr(), T, k, 160, x.data_ptr(), 160,
+                                       rows.data_ptr(), stream), "fmoe_permute_gather")
+    for a, b in zip(got, p):
+        assert torch.equal(a, b)
+    assert int(status) == (len(range(0, N, 5)) if bad else 0)
+
+
 @pytest.mark.parametrize("E,block", [(1024, 1024), (1025, 256)])  # rank + place; rank + scan + fill
 def test_ids_overwritten_after_ranking_write_nothing_outside(E, block):
     """The ids lie where the ranking kernel stores its ranks, so the kernel that places the slots

@@ -267,8 +267,10 @@ def test_metadata_and_slot_plan_in_one_call_equals_two_calls(E):
     np.testing.assert_array_equal(st1[:3], st2[:3])
 
 
+@pytest.mark.parametrize("small", [1, 2])  # the slot-map plan; the small path, which needs none
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_unpermute_with_permutation_is_bit_identical(dtype):
+def test_unpermute_with_permutation_is_bit_identical(dtype, small, kernel_options, library_calls):
+    kernel_options(small=small)
     T, D, E, k = 256, 192, 32, 6
     ids, w = _routing(T, E, k, seed=22)
     x = torch.randn(T, D).to(dtype).to(DEV)
@@ -278,6 +280,7 @@ def test_unpermute_with_permutation_is_bit_identical(dtype):
     go = torch.randn(1, T, D, generator=torch.Generator().manual_seed(3)).to(dtype).to(DEV)
     a = fastmoe_amd.unpermute(parts, p.reverse_map_indices, sw, (1, T), permutation=p)
     ga = torch.autograd.grad(a, [sw, *parts], go)
+    assert ("fmoe_build_metadata_and_plan_from_slots" in library_calls) == (small == 1)
     b = fastmoe_amd.unpermute(parts, p.reverse_map_indices, sw, (1, T))
     gb = torch.autograd.grad(b, [sw, *parts], go)
     assert torch.equal(a, b)
@@ -304,9 +307,11 @@ def test_plan_from_slots_with_inconsistent_slots_stays_in_bounds():
     assert torch.isfinite(out).all()
 
 
-def test_graph_capture_of_the_layer_data_path_replays():
-    """permute_tokens -> per-expert views -> unpermute with the slot-map plan, captured once as a
-    graph: every replay equals the eager result bit for bit."""
+@pytest.mark.parametrize("small", [1, 2])
+def test_graph_capture_of_the_layer_data_path_replays(small, kernel_options, library_calls):
+    """permute_tokens -> per-expert views -> unpermute with the slot-map plan (or on the small path),
+    captured once as a graph: every replay equals the eager result bit for bit."""
+    kernel_options(small=small)
     T, D, E, k = 256, 128, 16, 4
     ids, w = _routing(T, E, k, seed=31)
     x = torch.randn(T, D).to(torch.bfloat16).to(DEV)
@@ -321,6 +326,7 @@ def test_graph_capture_of_the_layer_data_path_replays():
 
     with torch.no_grad():
         eager = bits(step())
+        assert ("fmoe_build_metadata_and_plan_from_slots" in library_calls) == (small == 1)
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):

@@ -50,12 +50,20 @@ def _to_dev(experts, idx, w):
     return [x.to(DEV) for x in experts], idx.to(DEV), w.to(DEV)
 
 
+# The planned path and, for up to 4096 rows, the one-launch small path: values of the "small" option.
+_PATHS = {"planned": 1, "small": 2}
+
+
+@pytest.mark.parametrize("path", list(_PATHS))
 @pytest.mark.parametrize("name", list(SCALED))
-def test_fwd_det_bitexact(name):
+def test_fwd_det_bitexact(name, path, kernel_options, library_calls):
+    kernel_options(small=_PATHS[path])
     wl, T, idx, w, experts = _inputs(name)
     xd, idd, wd = _to_dev(experts, idx, w)
     out = fastmoe_amd.grouped_weighted_scatter_add(xd, idd, wd, (T, wl.D), mode="det")
     torch.cuda.synchronize()
+    small = path == "small" and idx.numel() <= 4096
+    assert library_calls[-1] == ("fmoe_combine_fwd_small" if small else "fmoe_combine_fwd")
     assert out.dtype == wl.dtype and out.shape == (T, wl.D)
     want, _, bad = oracle_fwd(experts, idx, w, T, wl.dtype)
     assert bad == 0
@@ -90,14 +98,16 @@ def test_fwd_atomic_within_reordering(name, mode, order, kernel_options):
         assert np.all(np.abs(got - want16) <= packed_tol(k, scale, wl.dtype))
 
 
-def test_fwd_fp32_atomic_vs_det_on_published_shape():
+def test_fwd_fp32_atomic_vs_det_on_published_shape(kernel_options, library_calls):
     """The reference's own bench shape (randint indices, fp32): det is bit-exact, atomic close."""
+    kernel_options(small=1)
     wl, T, idx, w, experts = _inputs("published")
     xd, idd, wd = _to_dev(experts, idx, w)
     det = torch.zeros(T, wl.D, device=DEV)
     atom = torch.zeros(T, wl.D, device=DEV)
     fastmoe_amd.grouped_weighted_scatter_add(xd, idd, wd, (T, wl.D), out=det, mode="det")
     fastmoe_amd.grouped_weighted_scatter_add(xd, idd, wd, (T, wl.D), out=atom, mode="atomic")
+    assert library_calls.count("fmoe_combine_fwd") == 2
     want, acc, _ = oracle_fwd(experts, idx, w, T, torch.float32)
     np.testing.assert_array_equal(bits(det), want.view(np.uint32))
     k = int(np.bincount(idx.numpy(), minlength=T).max())
@@ -148,7 +158,7 @@ def test_bwd_grad_x_bitexact_grad_w_close(name, variant, kernel_options):
 
 @pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 16384), (torch.float32, 4104),
                                      (torch.float16, 8200)])
-def test_bwd_grad_w_staged_equals_per_wave(dtype, D, kernel_options):
+def test_bwd_grad_w_staged_equals_per_wave(dtype, D, kernel_options, library_calls):
     """At U = 4 the grad_w pass shares grad_out through LDS for tokens of 1-8 rows and reads it
     per wave otherwise (longer segments, the out-of-range segment, or FMOE_GW_STAGED=0): both give
     the same bits, and both meet the oracle's 1e-6 bar.  Row lengths are not multiples of the LDS
@@ -168,10 +178,11 @@ def test_bwd_grad_w_staged_equals_per_wave(dtype, D, kernel_options):
     xd, idd, wd = _to_dev(experts, idx, w)
     got = {}
     for staged in ("1", "0"):
-        kernel_options(gw_staged=int(staged), bwd_u=4)
+        kernel_options(gw_staged=int(staged), bwd_u=4, small=1)
         wg = wd.clone().requires_grad_(True)
         out = fastmoe_amd.grouped_weighted_scatter_add(xd, idd, wg, (T, D))
         (got[staged],) = torch.autograd.grad(out, [wg], go.to(DEV))
+        assert library_calls[-1] == "fmoe_combine_bwd"  # not the small path's
     np.testing.assert_array_equal(bits(got["1"]), bits(got["0"]))
     _, want_gw = oracle_bwd(experts, idx, w, T, go)
     scale = abs_dot(experts, idx, go, T)
@@ -723,11 +734,13 @@ def test_plan_hot_token_matches_oracle(path, T, N, hot, idx_dtype, kernel_option
     np.testing.assert_array_equal(bits(out), want.view(np.uint32))
 
 
-def test_bwd_f16_grad_x_rounds_twice_like_the_reference():
+@pytest.mark.parametrize("path", list(_PATHS))
+def test_bwd_f16_grad_x_rounds_twice_like_the_reference(path, kernel_options):
     """f16 experts, fp32 gates: grad_X is the fp32 product rounded to fp32 and then to f16
     (index_select * w, then autograd's cast; ops.py:344-353).  The inputs include elements where
     rounding the exact product once to f16 gives another value, so a kernel that fuses the
     multiply and the conversion (one rounding) fails here."""
+    kernel_options(small=_PATHS[path])
     gen = torch.Generator().manual_seed(47)
     T, D, k, E = 1000, 1024, 2, 64
     N = T * k
@@ -801,14 +814,15 @@ def test_random_shapes_against_oracle(plan, kernel_options):
         assert np.all(err <= 1e-6 * scale + rtol * np.abs(want_gw) + 1e-30), label
 
 
-@pytest.mark.parametrize("bwd", ["split", "fused"])
-def test_random_misaligned_buffers_against_oracle(bwd, kernel_options):
+@pytest.mark.parametrize("bwd,path", [("split", "planned"), ("fused", "planned"),
+                                      ("split", "small")])
+def test_random_misaligned_buffers_against_oracle(bwd, path, kernel_options):
     """16 seeded random cases whose buffers sit at arbitrary element offsets of shared pools:
     every expert (some empty) a contiguous view at a random offset, grad_out and an in-place out
     at odd offsets with padded row strides.  Forward (autograd and in place, det) bit-exact,
     grad_X bit-exact and grad_w within 1e-6 of sum|terms|, with the backward's two passes or its
-    fused pass."""
-    kernel_options(bwd_fused=1 if bwd == "fused" else 0)
+    fused pass, or the small path's one."""
+    kernel_options(bwd_fused=1 if bwd == "fused" else 0, small=_PATHS[path])
     rng = np.random.default_rng(4242)
     dts = [torch.float32, torch.bfloat16, torch.float16]
     for case in range(16):
@@ -865,11 +879,13 @@ def test_random_misaligned_buffers_against_oracle(bwd, kernel_options):
                                       if want_ip.dtype == np.float32 else want_ip, err_msg=label)
 
 
-def test_random_inplace_against_oracle():
+@pytest.mark.parametrize("path", list(_PATHS))
+def test_random_inplace_against_oracle(path, kernel_options):
     """30 seeded random in-place calls (ops.py:389-390: accumulate into the given out): out in
     fp32, bf16 or f16 with random prior contents and sometimes a padded row stride; the
     deterministic mode bit-exact against the oracle started from out's values, the atomic mode
     (fp32 out) within the reordering bound."""
+    kernel_options(small=_PATHS[path])
     rng = np.random.default_rng(77)
     dts = [torch.float32, torch.bfloat16, torch.float16]
     for case in range(30):
@@ -1070,12 +1086,12 @@ def test_metadata_matches_closed_forms():
 
 
 @pytest.mark.parametrize("tile", [0, 44, 42, 28, 24, 18])
-def test_fwd_det_every_tile_shape(tile, kernel_options):
+def test_fwd_det_every_tile_shape(tile, kernel_options, library_calls):
     """The deterministic forward with each tile shape (option fwd_tile <U><R>: U vectors per lane
     per row, R rows per batch; 0 = the automatic choice by D and the rows per token) is the oracle's
     result bit for bit: segments of 1, 2 and 8 rows and ragged ones, D that the chunk divides and
     D that leaves a partial chunk, bf16 and fp32, overwrite and in-place accumulation."""
-    kernel_options(fwd_tile=tile)
+    kernel_options(fwd_tile=tile, small=1)  # the small path has no tiles
     gen = torch.Generator().manual_seed(400 + tile)
     for T, D, k, dt in [(300, 7168, 1, torch.bfloat16), (300, 7168, 2, torch.bfloat16),
                         (200, 3072, 8, torch.bfloat16), (257, 4104, 2, torch.bfloat16),
@@ -1099,6 +1115,7 @@ def test_fwd_det_every_tile_shape(tile, kernel_options):
         want, _, _ = oracle_fwd(experts, idx, w, T, dt, acc_init=init.float().numpy())
         np.testing.assert_array_equal(bits(acc), want.view(np.uint32) if want.dtype == np.float32
                                       else want, err_msg=label + " in place")
+    assert library_calls.count("fmoe_combine_fwd") == 12
 
 
 @pytest.mark.parametrize("D", [1, 256])
