@@ -805,10 +805,10 @@ def _combine_backward(ctx, grad_output, needs_w: bool, needs_x: Sequence[bool]):
                     gw_ptr, w_code, stream)
             _abi.check(rc, "fmoe_combine_bwd_small")
         elif gx_ptr and gw_ptr and _TIMER is not None and not _abi.option("bwd_fused"):
-            # Timed: the grad_X (write) and grad_w (read) passes, one call each -- the same two
-            # launches fmoe_combine_bwd makes when given both outputs, issued separately so that
-            # each gets its own span.
-            for name, a, b in (("bwd_gx", gx_ptr, None), ("bwd_gw", None, gw_ptr)):
+            # Timed: the grad_w (read) and grad_X (write) passes, one call each -- the same two
+            # launches, in the order, that fmoe_combine_bwd makes when given both outputs, issued
+            # separately so that each gets its own span.
+            for name, a, b in (("bwd_gw", None, gw_ptr), ("bwd_gx", gx_ptr, None)):
                 with _span(name):
                     rc = lib.fmoe_combine_bwd(plan, N, T, D, x_code, go.data_ptr(), g_code,
                                               g_stride, a, b, w_code, stream)

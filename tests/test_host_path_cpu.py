@@ -156,7 +156,7 @@ def test_autograd_forward_and_backward_calls(fake):
     assert kinds == ["metadata_plan", "fwd", "bwd"]
     assert fake.calls[0] == ("metadata_plan", 3, [3, 0, 5], 4, 32, _abi.I64, _abi.F32)
     assert fake.calls[1] == ("fwd", _abi.MODE_DET, 8, 4, 16, _abi.BF16, _abi.BF16, 16, 0)
-    # one call with both outputs (the library runs the grad_X pass, then the grad_w pass)
+    # one call with both outputs (the library runs the grad_w pass, then the grad_X pass)
     assert fake.calls[2] == ("bwd", 8, 4, 16, _abi.BF16, 16, True, True, _abi.F32)
     assert grads[0].shape == (N,) and grads[0].dtype == torch.float32
     assert [g.shape[0] for g in grads[1:]] == [3, 0, 5]
@@ -192,10 +192,10 @@ def test_timed_backward_issues_each_pass_in_its_own_span(fake, monkeypatch):
     w = torch.rand(8, requires_grad=True)
     out = fastmoe_amd.grouped_weighted_scatter_add(xs, torch.randint(0, 4, (8,)), w, (4, 16))
     torch.autograd.grad(out, [w, *xs], torch.ones(4, 16, dtype=torch.bfloat16))
-    assert timer.names == ["metadata_plan", "fwd_det", "bwd_gx", "bwd_gw"]
-    # grad_X pass, then grad_w pass
-    assert fake.calls[2] == ("bwd", 8, 4, 16, _abi.BF16, 16, True, False, _abi.F32)
-    assert fake.calls[3] == ("bwd", 8, 4, 16, _abi.BF16, 16, False, True, _abi.F32)
+    assert timer.names == ["metadata_plan", "fwd_det", "bwd_gw", "bwd_gx"]
+    # grad_w pass, then grad_X pass: the library's own order
+    assert fake.calls[2] == ("bwd", 8, 4, 16, _abi.BF16, 16, False, True, _abi.F32)
+    assert fake.calls[3] == ("bwd", 8, 4, 16, _abi.BF16, 16, True, False, _abi.F32)
 
 
 def test_fused_backward_is_one_call(fake):
