@@ -109,19 +109,22 @@ def _permute(x_flat, topk_weights, topk_indices, num_experts, validate):
     es = x_flat.element_size()
     out = torch.empty((N, D), dtype=x_flat.dtype, device=dev)
     x_stride = (x_flat.stride(0) if T > 1 else D) * es
-    whole = N > 0 and D > 0 and ops._TIMER is None  # one call; timed: one per span
+    small = N <= _small_slots()  # one launch
+    # one call; timed: one per span, of what an untimed call launches
+    whole = N > 0 and D > 0 and (small or ops._TIMER is None)
     ws = None
-    if not whole or N > _small_slots():
+    if not whole or not small:
         ws = torch.empty(max(lib.fmoe_permute_workspace_bytes(N, E), 256), dtype=torch.uint8,
                          device=dev)
     with _on_device(dev):
         if whole:
-            rc = lib.fmoe_permute(
-                ids.data_ptr(), _INDEX_CODES[ids.dtype], gates.data_ptr(),
-                _FLOAT_CODES[gates.dtype], T, k, E, D * es, x_flat.data_ptr(), x_stride,
-                counts.data_ptr(), offsets.data_ptr(), rev.data_ptr(), sorted_w.data_ptr(),
-                slot_pos.data_ptr(), status.data_ptr(), out.data_ptr(),
-                ws.data_ptr() if ws is not None else None, _stream_handle(dev))
+            with _span("permute"):
+                rc = lib.fmoe_permute(
+                    ids.data_ptr(), _INDEX_CODES[ids.dtype], gates.data_ptr(),
+                    _FLOAT_CODES[gates.dtype], T, k, E, D * es, x_flat.data_ptr(), x_stride,
+                    counts.data_ptr(), offsets.data_ptr(), rev.data_ptr(), sorted_w.data_ptr(),
+                    slot_pos.data_ptr(), status.data_ptr(), out.data_ptr(),
+                    ws.data_ptr() if ws is not None else None, _stream_handle(dev))
             _abi.check(rc, "fmoe_permute")
         else:
             with _span("permute_build"):

@@ -1,13 +1,14 @@
 """Host-side checks of the dispatch permutation and MoE layer API (CPU only, no kernel launch)."""
 from __future__ import annotations
 
+import contextlib
 import ctypes
 
 import pytest
 import torch
 
 import fastmoe_amd
-from fastmoe_amd import _abi
+from fastmoe_amd import _abi, dispatch, ops
 from fastmoe_amd.consts import MoEImplementation
 
 
@@ -64,3 +65,37 @@ def test_gather_and_gate_grad_reject_bad_arguments():
 def test_implementation_selector():
     assert MoEImplementation("fast") is MoEImplementation.FAST
     assert fastmoe_amd.MoEFeedForward(8, 16, 2, 1, "standard").implementation == "standard"
+
+
+@pytest.mark.parametrize("T,D,untimed,timed", [
+    (4, 8, ["fmoe_permute"], ["permute"]),                       # the one launch: one span
+    (2048, 8, ["fmoe_permute"], ["permute"]),                    # 4096 slots
+    (2049, 8, ["fmoe_permute"], ["permute_build", "permute_gather"]),
+    (4, 0, ["fmoe_permute_build"], ["permute_build"]),           # no rows to copy
+])
+def test_timed_permutation_times_what_an_untimed_one_launches(T, D, untimed, timed, monkeypatch):
+    calls, spans = [], []
+
+    class Lib:
+        fmoe_permute_small_max_slots = _abi.lib().fmoe_permute_small_max_slots
+        fmoe_permute_workspace_bytes = _abi.lib().fmoe_permute_workspace_bytes
+
+        def __getattr__(self, name):
+            return lambda *args: calls.append(name) or 0
+
+    class Timer:
+        def span(self, name):
+            spans.append(name)
+            return contextlib.nullcontext()
+
+    lib = Lib()
+    monkeypatch.setattr(_abi, "lib", lambda: lib)
+    monkeypatch.setattr(dispatch, "_stream_handle", lambda dev: 0)
+    monkeypatch.setattr(dispatch, "_on_device", lambda dev: contextlib.nullcontext())
+    args = (torch.zeros(T, D), torch.rand(T, 2), torch.zeros(T, 2, dtype=torch.long), 4, False)
+    dispatch._permute(*args)
+    assert calls == untimed
+    calls.clear()
+    monkeypatch.setattr(ops, "_TIMER", Timer())
+    dispatch._permute(*args)
+    assert spans == timed and calls == ["fmoe_" + name for name in timed]
