@@ -502,7 +502,8 @@ __global__ __launch_bounds__(kFewThreads) void k_fwd_atomic_few(
 #pragma unroll
   for (int j = 0; j < kFewRows / kFewThreads; ++j)
     if (tok[j] >= 0)
-      list[atomicAdd(&place[tok[j]], 1)] = (uint32_t)tok[j] << 16 | (uint32_t)(tid + j * kFewThreads);
+      list[atomicAdd(&place[tok[j]], 1)] =
+          (uint32_t)tok[j] << 16 | (uint32_t)(tid + j * kFewThreads);
   __syncthreads();
 
   const uint32_t row_bytes = D * (uint32_t)sizeof(TX);
@@ -757,9 +758,9 @@ struct FwdArgs {
 // So a forward whose backward follows streams from 96 MiB, and one alone only from 7 rows per token,
 // where it gains as much in a program that goes on to other buffers as it loses in one that does not.
 // Steps below that line (2048, 16384, top-8, 64 MiB: 313.7 -> 297.5 us) stay temporal with the
-// forwards.  An accumulating call has just read its output and the caller has just
-// written it, so its lines are in the cache: fp32, 256 MiB, zero-fill + call 291.6 us temporal,
-// 316.9 us non-temporal; it stays temporal.
+// forwards.  An accumulating call has just read its output and the caller has just written it, so its
+// lines are in the cache: fp32, 256 MiB, zero-fill + call 291.6 us temporal, 316.9 us non-temporal;
+// it stays temporal.
 static int streams_out(const FwdArgs& a, int64_t elem_bytes) {
   return !a.accumulate && a.T * a.D * elem_bytes >= FMOE_STREAM_OUT_BYTES &&
          (a.step || a.N >= 7 * a.T);
@@ -772,9 +773,9 @@ static int launch_fwd_k(const FwdArgs& a, int64_t chunks) {
     if (int rc = grid_for(a.T * chunks, "fmoe_combine_fwd(det)", &blocks)) return rc;
     const int persist = (int)fmoe_host::opt(fmoe_host::kOptFwdGrid);  // 0 = one wave per unit
     if (persist > 0 && (unsigned)persist < blocks) blocks = (unsigned)persist;
-    hipLaunchKernelGGL((k_fwd_det<TX, TO, V, U, RB>), dim3(blocks), dim3(kGroup), a.lds, a.s, a.status,
-                       a.row_ptr, a.rec, static_cast<TO*>(a.out), a.out_stride, (uint32_t)a.D,
-                       (uint32_t)a.T, (uint32_t)chunks, a.accumulate,
+    hipLaunchKernelGGL((k_fwd_det<TX, TO, V, U, RB>), dim3(blocks), dim3(kGroup), a.lds, a.s,
+                       a.status, a.row_ptr, a.rec, static_cast<TO*>(a.out), a.out_stride,
+                       (uint32_t)a.D, (uint32_t)a.T, (uint32_t)chunks, a.accumulate,
                        streams_out(a, sizeof(TO)));
     return fmoe_host::check_launch("fmoe_combine_fwd(det)");
   }
@@ -1016,7 +1017,13 @@ struct SlotsBwdArgs {
 // always followed by more passes over as much data, which pay for the lines left in the cache.
 // Permutation forward + backward, three sets of buffers in turn, bf16, temporal / non-temporal:
 // T=8192, D=4096, top-6 and T=4096, D=8192, top-6 (64 MiB) 180.9 / 165.9 and 182.0 / 164.8 us;
-// 28 and 32 MiB of grad_x make no difference.
+// 28 and 32 MiB of grad_x make no difference.  Where the program frees each result at once, so that
+// the next call's buffers are the same lines, forward + backward hardly changes up to 128 MiB and
+// gains beyond -- time non-temporal / temporal at top-1, 2, 4, 6, 8:
+//   8192, 4096 (64 MiB)    0.98, 0.63, 0.91, 0.99, 1.00     16384, 4096 (128 MiB)  1.00, 1.04, 1.01,
+//   12288, 4096 (96 MiB)   0.98, 0.99, 1.00, 1.00, 1.01                            1.02, 1.01
+//   16384, 7168 (224 MiB)  0.95, 0.96, 0.96, 0.98, 0.98     16384, 16384 (512 MiB) 0.95, 0.95, 0.95
+// (the backward alone, over and over, loses 2 to 5 % there, and 5 to 19 % at 224 MiB).
 constexpr int64_t kSlotsStreamBytes = int64_t(48) << 20;
 
 template <typename TX, int V, int U, int RB, bool GATES, typename TG>

@@ -330,10 +330,10 @@ __device__ __forceinline__ void copy_row(rsrc_t rs, rsrc_t rd, uint32_t row_byte
 // row.  Expert e's first row is the number of values below e << 16; those E + 1 counts are spread
 // over the waves of the grid, which has a wave for every slot or every count, whichever are more (in
 // a graph, N=1, E=4096: 3.2 us, the launches that this replaces 15.4, and 186 with a grid for the
-// slots alone; N=8, E=256: 3.7, 10.0 and 14.8).  Staging reads the N ids once per workgroup from L2, so the gain over
-// rank + place + gather shrinks with N (one MI355X, top-8, E=256, D=7168, bf16, us): N=128 14.1 ->
-// 8.1, N=1024 14.4 -> 9.1, N=2048 16.7 -> 11.1, N=4096 22.4 -> 17.4, where the rows' own copy is
-// most of it.
+// slots alone; N=8, E=256: 3.7, 10.0 and 14.8).  Staging reads the N ids once per workgroup from L2,
+// so the gain over rank + place + gather shrinks with N (one MI355X, top-8, E=256, D=7168, bf16, us):
+// N=128 14.1 -> 8.1, N=1024 14.4 -> 9.1, N=2048 16.7 -> 11.1, N=4096 22.4 -> 17.4, where the rows' own
+// copy is most of it.
 constexpr int kPermSmallSlots = 4096;
 constexpr int kPermSmallWaves = 8;
 constexpr unsigned kPermSmallGroups = 1024;
@@ -376,9 +376,8 @@ __global__ __launch_bounds__(kPermSmallWaves * kWave) void k_perm_small(
       sorted_gates[pos] = gates[i];
       slot_pos[i] = (int32_t)pos;
     }
-    if (row_bytes)  // wave-uniform
-      copy_row<VB>(make_rsrc(x + (int64_t)t * x_stride_bytes, row_bytes),
-                   make_rsrc(out + (int64_t)pos * row_bytes, row_bytes), row_bytes, lane);
+    copy_row<VB>(make_rsrc(x + (int64_t)t * x_stride_bytes, row_bytes),
+                 make_rsrc(out + (int64_t)pos * row_bytes, row_bytes), row_bytes, lane);
   }
   for (uint32_t e = first; e <= E; e += waves) {
     const int lo = count_below(v, n4, e << 16, lane);
@@ -402,7 +401,7 @@ __global__ __launch_bounds__(kPermGatherWaves * kWave) void k_perm_gather(
   const rsrc_t rs = make_rsrc(x + t * x_stride_bytes, row_bytes);
   for (int64_t j = wave; j < k; j += kPermGatherWaves) {
     const int64_t pos = slot_pos[t * k + j];
-    if (pos < 0 || pos >= N) continue;  // slot_pos comes from fmoe_permute_build: always in range
+    if (pos < 0 || pos >= N) continue;  // a slot map of fmoe_permute_build is in range; any may come
     copy_row<VB>(rs, make_rsrc(out + pos * (int64_t)row_bytes, row_bytes), row_bytes, lane);
   }
 }
