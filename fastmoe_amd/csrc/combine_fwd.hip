@@ -1019,11 +1019,13 @@ struct SlotsBwdArgs {
 // T=8192, D=4096, top-6 and T=4096, D=8192, top-6 (64 MiB) 180.9 / 165.9 and 182.0 / 164.8 us;
 // 28 and 32 MiB of grad_x make no difference.  Where the program frees each result at once, so that
 // the next call's buffers are the same lines, forward + backward hardly changes up to 128 MiB and
-// gains beyond -- time non-temporal / temporal at top-1, 2, 4, 6, 8:
-//   8192, 4096 (64 MiB)    0.98, 0.63, 0.91, 0.99, 1.00     16384, 4096 (128 MiB)  1.00, 1.04, 1.01,
-//   12288, 4096 (96 MiB)   0.98, 0.99, 1.00, 1.00, 1.01                            1.02, 1.01
-//   16384, 7168 (224 MiB)  0.95, 0.96, 0.96, 0.98, 0.98     16384, 16384 (512 MiB) 0.95, 0.95, 0.95
-// (the backward alone, over and over, loses 2 to 5 % there, and 5 to 19 % at 224 MiB).
+// gains beyond; time non-temporal / temporal where the GPU bounds the call:
+//   8192, 4096 (64 MiB)    top-6 0.99, top-8 1.00
+//   12288, 4096 (96 MiB)   top-4 1.00, top-6 1.00, top-8 1.01
+//   16384, 4096 (128 MiB)  top-2 1.04, top-4 1.01, top-6 1.02, top-8 1.01
+//   16384, 7168 (224 MiB)  top-1 0.95, top-2 0.96, top-4 0.96, top-6 0.98, top-8 0.98
+//   16384, 16384 (512 MiB) top-1 0.95, top-2 0.95, top-4 0.95
+// (the backward alone, over and over, loses 2 to 5 % there, and 3 to 19 % at 224 MiB).
 constexpr int64_t kSlotsStreamBytes = int64_t(48) << 20;
 
 template <typename TX, int V, int U, int RB, bool GATES, typename TG>
