@@ -140,10 +140,17 @@ def kernel_bytes(T: int, D: int, N: int, x_bytes: int, out_bytes: int,
     bwd                  : both gradients in one pass (as ``algorithmic_bytes``)
     fwd_small, bwd_small : the one-launch small path's forward and backward (as fwd_det, bwd)
     permute_gather       : read x (T*D) + write the packed rows (N*D) + read slot_pos per slot
+    permute              : the one-launch permutation: as permute_gather, and per slot read the id
+                           and the gate, write the reverse map, the sorted gate and slot_pos
+    permute_backward     : read the packed rows' gradient (N*D) + write grad_x (T*D); per slot read
+                           slot_pos and a gate gradient, write one
     """
     fwd, bwd = algorithmic_bytes(T, D, N, x_bytes, out_bytes, gate_bytes)
+    rows = T * D * x_bytes + N * D * x_bytes
     return {
-        "permute_gather": T * D * x_bytes + N * D * x_bytes + N * 4,
+        "permute_gather": rows + N * 4,
+        "permute": rows + N * (8 + 8 + 4 + 2 * gate_bytes),
+        "permute_backward": rows + N * (4 + 2 * gate_bytes),
         "fwd_det": fwd,
         "fwd_atomic": fwd,
         "bwd_gx": T * D * x_bytes + N * D * x_bytes + N * (8 + gate_bytes),

@@ -99,3 +99,16 @@ def test_timed_permutation_times_what_an_untimed_one_launches(T, D, untimed, tim
     monkeypatch.setattr(ops, "_TIMER", Timer())
     dispatch._permute(*args)
     assert spans == timed and calls == ["fmoe_" + name for name in timed]
+
+
+def test_every_span_of_the_permutation_has_its_bytes():
+    """bench.py takes its dominant kernel from the spans that kernel_bytes knows: a small permutation
+    has the one span "permute" in its forward, any its backward's."""
+    from fastmoe_amd.workloads import kernel_bytes
+
+    T, D, k = 256, 512, 2
+    got = kernel_bytes(T, D, T * k, 4, 4)
+    rows = (T + T * k) * D * 4
+    assert got["permute"] == rows + T * k * (8 + 4 + 8 + 4 + 4)
+    assert got["permute_backward"] == rows + T * k * (4 + 4 + 4)
+    assert got["permute_gather"] == rows + T * k * 4
